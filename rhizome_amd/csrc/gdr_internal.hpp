@@ -14,6 +14,11 @@ namespace rhz {
 // Token-sequential fp32 recurrence over a dense or packed batch.
 hipError_t launch_recurrent(const rhz_gdr_prefill_args& a, hipStream_t stream);
 
+// The fp32-input prefill in 16-token chunks on fp32 MFMA, where the call's
+// shape and alignment allow it.
+bool chunk32_supported(const rhz_gdr_prefill_args& a);
+hipError_t launch_chunk32(const rhz_gdr_prefill_args& a, hipStream_t stream);
+
 // One decode position for every (b, h), state in place.
 hipError_t launch_decode(const rhz_gdr_decode_args& a, hipStream_t stream);
 

@@ -421,6 +421,8 @@ hipError_t launch_multistep(const rhz_gdr_multistep_args& a, hipStream_t st) {
 }
 
 hipError_t launch_recurrent(const rhz_gdr_prefill_args& a, hipStream_t st) {
+    // AUTO leaves the form to the library: the chunked one wherever it applies
+    if (a.algo == RHZ_ALGO_AUTO && chunk32_supported(a)) return launch_chunk32(a, st);
     SeqParams sp{a.q, a.k, a.v, a.gate, a.beta, a.cu_seqlens, a.initial_state, a.final_state, a.o,
                  a.seq_len, a.heads, a.d_k, a.d_v, a.gate_kind == RHZ_GATE_ALPHA};
     const int units = a.batch * a.heads;

@@ -1,0 +1,155 @@
+"""The fp32-input prefill's chunked form (what AUTO takes for fp32) against the
+f64 oracle and against the token-sequential recurrence, at the sizes where
+its tiles, its pipeline and its domain checks can go wrong.
+
+The tolerance is the fp32 path's (rtol 1e-4, atol 1e-4 RMS).
+"""
+import numpy as np
+import pytest
+import torch
+
+from gdr_cases import F32_TOL, Prefill, check_close
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(w, o, fin, tag):
+    ref_o, ref_f = w.oracle()
+    mo = check_close(o.cpu().numpy(), ref_o, F32_TOL, f"{tag} o")
+    mf = check_close(fin.cpu().numpy(), ref_f, F32_TOL, f"{tag} final state")
+    print(f"{tag}: o {mo['normwise']:.2e}  final {mf['normwise']:.2e}", flush=True)
+    return mo, mf
+
+
+# chunks of 16 tokens, superblocks of 4 chunks, tiles of 32 rows, key widths
+# padded to 32, 64 and 128, value tiles that end inside a scan wave's 16 rows
+SHAPES = [
+    dict(batch=1, heads=1, seq_len=1, d_k=4, d_v=4),
+    dict(batch=2, heads=3, seq_len=15, d_k=32, d_v=32),
+    dict(batch=1, heads=2, seq_len=16, d_k=20, d_v=36),
+    dict(batch=3, heads=1, seq_len=17, d_k=64, d_v=64),
+    dict(batch=1, heads=5, seq_len=63, d_k=36, d_v=12),
+    dict(batch=1, heads=2, seq_len=65, d_k=100, d_v=52),
+    dict(batch=2, heads=2, seq_len=129, d_k=128, d_v=128),
+    dict(batch=1, heads=9, seq_len=200, d_k=128, d_v=256),
+    dict(lengths=[0, 1, 16, 0, 31, 64, 200, 5, 0], heads=2, d_k=128, d_v=96, state_std=0.5),
+    dict(lengths=[33, 79, 128], heads=3, d_k=64, d_v=32, state_std=0.02),
+    dict(batch=1, heads=1, seq_len=3000, d_k=128, d_v=32, g_mean=-2.0, state_std=0.02),
+    dict(batch=1, heads=2, seq_len=500, d_k=32, d_v=64, g_mean=5.0),
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: ",".join(f"{k}={v}" for k, v in s.items()).replace(" ", ""))
+def test_shapes(device, shape):
+    w = Prefill(dtype=torch.float32, device=device, **shape)
+    o, fin = w.run()
+    mo, mf = _check(w, o, fin, str(shape))
+    if w.d_k >= 64 and w.n_tok >= 1000:
+        # no less accurate than the recurrence
+        ro, rf = w.run(algo="recurrent")
+        ref_o, ref_f = w.oracle()
+        for x, y, ref in ((o, ro, ref_o), (fin, rf, ref_f)):
+            e, er = (np.linalg.norm(t.double().cpu().numpy() - ref) for t in (x, y))
+            assert e <= 1.05 * er, (e, er)
+
+
+def test_unaligned_and_odd_shapes_keep_the_recurrence(device):
+    """Widths that are no multiple of 4, and v 4 bytes off 16-byte alignment."""
+    w = Prefill(batch=1, heads=2, seq_len=50, d_k=30, d_v=10, dtype=torch.float32, device=device)
+    _check(w, *w.run(), "d_k 30, d_v 10")
+    w = Prefill(batch=1, heads=2, seq_len=50, d_k=32, d_v=32, dtype=torch.float32, device=device)
+    buf = torch.empty(w.v.numel() + 1, device=device)
+    buf[1:] = w.v.flatten()
+    w.v = buf[1:].reshape(w.v.shape)
+    _check(w, *w.run(), "v off alignment")
+
+
+@pytest.mark.parametrize("m", [1, 16, 21, 64])
+def test_reset_forgets_history(device, m):
+    """alpha = 0 at position m: outputs from m on and final states are the same
+    numbers whatever came before."""
+    import rhizome_amd
+
+    w = Prefill(batch=2, heads=2, seq_len=90, d_k=128, d_v=32, dtype=torch.float32, device=device, state_std=0.5)
+    h = Prefill(batch=2, heads=2, seq_len=90, d_k=128, d_v=32, dtype=torch.float32, device=device, state_std=0.02,
+                seed=1)
+
+    def run(a, b):
+        mix = [torch.cat([w.shaped(x)[:, :m], w.shaped(y)[:, m:]], 1).contiguous()
+               for x, y in ((a.q, b.q), (a.k, b.k), (a.v, b.v), (torch.exp(a.g), torch.exp(b.g)), (a.beta, b.beta))]
+        mix[3][:, m] = 0.0
+        return rhizome_amd.prefill(mix[0], mix[1], mix[2], None, mix[4], alpha=mix[3], initial_state=a.init)
+
+    (o1, f1), (o2, f2) = run(w, w), run(h, w)
+    assert torch.equal(o1[:, m:], o2[:, m:]) and torch.equal(f1, f2)
+    assert not torch.equal(o1[:, :m], o2[:, :m])
+
+
+def _leave(w, case, t, h):
+    if case == "beta |k|^2 above 2":
+        w.k[t, h] *= 3.0
+    elif case == "beta -0.5":
+        w.beta[t, h] = -0.5
+    elif case == "alpha 1.05":
+        w.g[t, h] = float(np.log(1.05))
+    elif case == "v inf":
+        w.v[t, h, 3] = float("inf")
+    elif case == "v nan in the second row half":
+        w.v[t, h, 20] = float("nan")
+    elif case == "q nan":
+        w.q[t, h, 5] = float("nan")
+    elif case == "k nan":
+        w.k[t, h, 1] = float("nan")
+    elif case == "beta nan":
+        w.beta[t, h] = float("nan")
+    elif case == "gate nan":
+        w.g[t, h] = float("nan")
+    elif case == "v 3e38":  # finite, but its sums overflow
+        w.v[t - 8:t + 6, h, 40] = 3e38
+    else:
+        raise ValueError(case)
+
+
+CASES = ["beta |k|^2 above 2", "beta -0.5", "alpha 1.05", "v inf", "v nan in the second row half", "q nan", "k nan",
+         "beta nan", "gate nan", "v 3e38"]
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("case", CASES)
+def test_out_of_domain_is_the_recurrence(device, case, in_place):
+    """Inputs outside the op's domain or not finite, at the last token of a
+    16-token chunk or at the first of a partial one, in one head: every other
+    (sequence, head) is unchanged, and the head's tiles equal the recurrence
+    bit for bit or the chunked result where they hold no such value (a value
+    row's tile), also when the state is updated in place."""
+    kw = dict(heads=2, d_k=128, d_v=64, lengths=[47, 70], dtype=torch.float32, device=device, state_std=0.1)
+    w, plain = Prefill(**kw), Prefill(**kw)
+    if "3e38" in case:
+        w.q *= 1e3
+        plain.q *= 1e3
+    _leave(w, case, 47 + 31 if "row" in case else 47 + 64, 1)
+    want_o, want_f = plain.run()
+
+    def run(**k):
+        import rhizome_amd
+
+        init = w.init.clone()
+        fin = init if in_place else None
+        return rhizome_amd.prefill(w.q, w.k, w.v, w.g, w.beta, cu_seqlens=w.cu_dev, initial_state=init,
+                                   final_state=fin, **k)
+
+    (o, f), (ro, rf) = run(), run(algo="recurrent")
+    bits = lambda x: x.contiguous().view(torch.int32)  # noqa: E731  (NaN compares equal to itself)
+    other = torch.ones(o.shape[:2], dtype=torch.bool, device=device)
+    other[47:, 1] = False
+    assert torch.equal(o[other], want_o[other]) and torch.equal(f[0], want_f[0]) and torch.equal(f[1, 0], want_f[1, 0])
+    touched = 0
+    for i0 in (0, 32):  # the head's two tiles
+        a, r = o[47:, 1, i0:i0 + 32], ro[47:, 1, i0:i0 + 32]
+        fa, fr = f[1, 1, i0:i0 + 32], rf[1, 1, i0:i0 + 32]
+        same = torch.equal(torch.isnan(a), torch.isnan(r)) and torch.equal(bits(a.nan_to_num()), bits(r.nan_to_num())) \
+            and torch.equal(bits(fa.nan_to_num()), bits(fr.nan_to_num()))
+        touched += same
+        if not same:  # a tile without the value: the chunked result
+            assert torch.equal(a, want_o[47:, 1, i0:i0 + 32]) and torch.equal(fa, want_f[1, 1, i0:i0 + 32])
+    assert touched >= 1
