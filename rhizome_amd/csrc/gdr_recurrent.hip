@@ -273,11 +273,15 @@ __global__ __launch_bounds__(64) void gdr_recurrent_kernel(SeqParams p) {
 // waves per (sequence, head, 4 * 64 / LPR rows), running staged_rows
 // (gdr_staged.hpp).  The global loads of a block have a whole block's
 // compute to arrive.
+// Sequences of more than max_len tokens are left out.
 template <int LPR, typename T, int VPL, int NW>
-__global__ __launch_bounds__(NW * 64) void gdr_staged_recurrent_kernel(SeqParams p) {
+__global__ __launch_bounds__(NW * 64) void gdr_staged_recurrent_kernel(SeqParams p, int max_len) {
     __shared__ __align__(16) StageSmem<LPR, VPL, NW> sm;
     const int unit = blockIdx.x;
     const int seq = unit / p.heads, h = unit % p.heads;
+    int t0, t1;
+    seq_bounds(p.cu_seqlens, seq, p.seq_len, t0, t1);
+    if (t1 - t0 > max_len) return;  // uniform
     staged_rows<LPR, T, VPL, NW>(p, sm, seq, h, blockIdx.y * StageSmem<LPR, VPL, NW>::RPB, threadIdx.x);
 }
 
@@ -380,19 +384,26 @@ hipError_t staged_pick_lpr(const SeqParams& sp, int units, int dk, int dv, hipSt
         // other's latency along the position chain.
         using Sh = StageShape<16, 8, 8>;
         dim3 grid(units, (dv + Sh::RPB - 1) / Sh::RPB);
-        hipLaunchKernelGGL((gdr_staged_recurrent_kernel<16, T, 8, 8>), grid, dim3(Sh::THREADS), 0, st, sp);
+        hipLaunchKernelGGL((gdr_staged_recurrent_kernel<16, T, 8, 8>), grid, dim3(Sh::THREADS), 0, st, sp, INT32_MAX);
         return hipGetLastError();
     }
     const int rpb = kStageWaves * (64 / lpr);
     dim3 grid(units, (dv + rpb - 1) / rpb);
     switch (lpr) {
-        case 2: hipLaunchKernelGGL((gdr_staged_recurrent_kernel<2, T, 16, kStageWaves>), grid, dim3(kStageThreads), 0, st, sp); break;
-        default: hipLaunchKernelGGL((gdr_staged_recurrent_kernel<4, T, 16, kStageWaves>), grid, dim3(kStageThreads), 0, st, sp); break;
+        case 2: hipLaunchKernelGGL((gdr_staged_recurrent_kernel<2, T, 16, kStageWaves>), grid, dim3(kStageThreads), 0, st, sp, INT32_MAX); break;
+        default: hipLaunchKernelGGL((gdr_staged_recurrent_kernel<4, T, 16, kStageWaves>), grid, dim3(kStageThreads), 0, st, sp, INT32_MAX); break;
     }
     return hipGetLastError();
 }
 
 }  // namespace
+
+hipError_t launch_staged_short(const SeqParams& sp, int units, int max_len, hipStream_t st) {
+    using Sh = StageShape<16, 8, 8>;
+    dim3 grid(units, (sp.d_v + Sh::RPB - 1) / Sh::RPB);
+    hipLaunchKernelGGL((gdr_staged_recurrent_kernel<16, float, 8, 8>), grid, dim3(Sh::THREADS), 0, st, sp, max_len);
+    return hipGetLastError();
+}
 
 hipError_t launch_decode(const rhz_gdr_decode_args& a, hipStream_t st) {
     StepParams sp{a.q, a.k, a.v, a.gate, a.beta, a.state, a.o, a.d_k, a.d_v, a.gate_kind == RHZ_GATE_ALPHA};

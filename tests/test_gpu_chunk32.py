@@ -25,15 +25,19 @@ def _check(w, o, fin, tag):
 # padded to 32, 64 and 128, value tiles that end inside a scan wave's 16 rows
 SHAPES = [
     dict(batch=1, heads=1, seq_len=1, d_k=4, d_v=4),
-    dict(batch=2, heads=3, seq_len=15, d_k=32, d_v=32),
-    dict(batch=1, heads=2, seq_len=16, d_k=20, d_v=36),
-    dict(batch=3, heads=1, seq_len=17, d_k=64, d_v=64),
-    dict(batch=1, heads=5, seq_len=63, d_k=36, d_v=12),
+    dict(batch=2, heads=3, seq_len=79, d_k=32, d_v=32),
+    dict(batch=1, heads=2, seq_len=80, d_k=20, d_v=36),
+    dict(batch=3, heads=1, seq_len=81, d_k=64, d_v=64),
+    dict(batch=1, heads=5, seq_len=127, d_k=36, d_v=12),
+    dict(batch=1, heads=5, seq_len=64, d_k=36, d_v=12),
     dict(batch=1, heads=2, seq_len=65, d_k=100, d_v=52),
     dict(batch=2, heads=2, seq_len=129, d_k=128, d_v=128),
     dict(batch=1, heads=9, seq_len=200, d_k=128, d_v=256),
     dict(lengths=[0, 1, 16, 0, 31, 64, 200, 5, 0], heads=2, d_k=128, d_v=96, state_std=0.5),
     dict(lengths=[33, 79, 128], heads=3, d_k=64, d_v=32, state_std=0.02),
+    # few tokens per sequence on average: the short ones in the recurrence's kernel
+    dict(lengths=[64, 65, 0, 3, 100, 7, 1, 64, 130, 33], heads=2, d_k=128, d_v=40, state_std=0.3),
+    dict(lengths=[5, 40], heads=2, d_k=32, d_v=64),
     dict(batch=1, heads=1, seq_len=3000, d_k=128, d_v=32, g_mean=-2.0, state_std=0.02),
     dict(batch=1, heads=2, seq_len=500, d_k=32, d_v=64, g_mean=5.0),
 ]
@@ -64,14 +68,34 @@ def test_unaligned_and_odd_shapes_keep_the_recurrence(device):
     _check(w, *w.run(), "v off alignment")
 
 
+@pytest.mark.parametrize("d_k", [32, 128])
+def test_batch_invariant(device, d_k):
+    """A sequence gives the same bits alone, in a pack of long sequences and in
+    a pack whose average is short (which is launched in two parts)."""
+    import rhizome_amd
+
+    w = Prefill(lengths=[64, 200, 65, 17], heads=2, d_k=d_k, d_v=64, dtype=torch.float32, device=device,
+                state_std=0.3)
+    o, f = w.run()
+    at = [(int(a), int(b)) for a, b in zip(w.cu[:-1], w.cu[1:])]
+    for i, (a, b) in enumerate(at):
+        for tail in (0, 80):  # alone, and followed by 80 empty sequences
+            cu = torch.tensor([0, b - a] + [b - a] * tail, dtype=torch.int32, device=device)
+            init = torch.cat([w.init[i:i + 1]] + [w.init[:1]] * tail)
+            o1, f1 = rhizome_amd.prefill(w.q[a:b], w.k[a:b], w.v[a:b], w.g[a:b], w.beta[a:b], cu_seqlens=cu,
+                                         initial_state=init)
+            assert torch.equal(o1, o[a:b]) and torch.equal(f1[0], f[i])
+            assert tail == 0 or torch.equal(f1[1:], init[1:])
+
+
 @pytest.mark.parametrize("m", [1, 16, 21, 64])
 def test_reset_forgets_history(device, m):
     """alpha = 0 at position m: outputs from m on and final states are the same
     numbers whatever came before."""
     import rhizome_amd
 
-    w = Prefill(batch=2, heads=2, seq_len=90, d_k=128, d_v=32, dtype=torch.float32, device=device, state_std=0.5)
-    h = Prefill(batch=2, heads=2, seq_len=90, d_k=128, d_v=32, dtype=torch.float32, device=device, state_std=0.02,
+    w = Prefill(batch=2, heads=2, seq_len=150, d_k=128, d_v=32, dtype=torch.float32, device=device, state_std=0.5)
+    h = Prefill(batch=2, heads=2, seq_len=150, d_k=128, d_v=32, dtype=torch.float32, device=device, state_std=0.02,
                 seed=1)
 
     def run(a, b):
@@ -122,12 +146,12 @@ def test_out_of_domain_is_the_recurrence(device, case, in_place):
     (sequence, head) is unchanged, and the head's tiles equal the recurrence
     bit for bit or the chunked result where they hold no such value (a value
     row's tile), also when the state is updated in place."""
-    kw = dict(heads=2, d_k=128, d_v=64, lengths=[47, 70], dtype=torch.float32, device=device, state_std=0.1)
+    kw = dict(heads=2, d_k=128, d_v=64, lengths=[47, 102], dtype=torch.float32, device=device, state_std=0.1)
     w, plain = Prefill(**kw), Prefill(**kw)
     if "3e38" in case:
         w.q *= 1e3
         plain.q *= 1e3
-    _leave(w, case, 47 + 31 if "row" in case else 47 + 64, 1)
+    _leave(w, case, 47 + 31 if "row" in case else 47 + 96, 1)
     want_o, want_f = plain.run()
 
     def run(**k):
