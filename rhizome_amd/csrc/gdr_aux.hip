@@ -115,6 +115,51 @@ __device__ __forceinline__ int seq_end(const ConvParams& p, int s) {
     return min(max(p.cu[s + 1], seq_start(p, s)), p.seq_len);
 }
 
+// The carried state of N consecutive channels, [channel][3] (base: index of
+// the first value): 16-byte accesses where N channels are 3 N / 4 whole ones.
+template <int N>
+__device__ __forceinline__ void load_conv_state(const float* init, long base, float (&st)[N][3]) {
+    if constexpr (N % 4 == 0) {
+        if (aligned16(init)) {  // uniform
+            float f[3 * N];
+#pragma unroll
+            for (int i = 0; i < 3 * N / 4; ++i) {
+                const f32x4 x = reinterpret_cast<const f32x4*>(init + base)[i];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) f[4 * i + j] = x[j];
+            }
+#pragma unroll
+            for (int e = 0; e < N; ++e)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) st[e][k] = f[3 * e + k];
+            return;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) st[e][k] = init[base + 3 * e + k];
+}
+template <int N>
+__device__ __forceinline__ void store_conv_state(float* fin, long base, const float (&a)[3][N]) {
+    if constexpr (N % 4 == 0) {
+        if (aligned16(fin)) {  // uniform
+#pragma unroll
+            for (int i = 0; i < 3 * N / 4; ++i) {
+                f32x4 x;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[j] = a[(4 * i + j) % 3][(4 * i + j) / 3];
+                reinterpret_cast<f32x4*>(fin + base)[i] = x;
+            }
+            return;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) fin[base + 3 * e + k] = a[k][e];
+}
+
 // Grid: one dimension, block b = (span b / ncb, channel block b % ncb);
 // each thread owns N consecutive channels (one 16-byte access per token
 // when VEC).  The span's outputs go to emit(t, c, y[N]), called for every
@@ -122,13 +167,13 @@ __device__ __forceinline__ int seq_end(const ConvParams& p, int s) {
 // of the block at once (the tokens are the block's, so the calls stay
 // converged across the block).
 template <typename T, bool VEC, int SPAN, typename Emit>
-__device__ __forceinline__ void conv_span(const ConvParams& p, int total, int ncb, Emit&& emit) {
+__device__ __forceinline__ void conv_span(const ConvParams& p, int total, int ncb, int span, Emit&& emit) {
     using V = Vec<T, VEC>;
     constexpr int N = V::N;
     const int c = ((blockIdx.x % ncb) * 256 + threadIdx.x) * N;
-    const int t0 = (blockIdx.x / ncb) * SPAN;
+    const int t0 = (blockIdx.x / ncb) * span;
     if (c >= p.C || t0 >= total) return;
-    const int t1 = min(t0 + SPAN, total);
+    const int t1 = min(t0 + span, total);
     const T* __restrict__ x = static_cast<const T*>(p.x);  // the outputs never overlap x
     const long C = p.C;
     float w[N][4], b[N];
@@ -179,31 +224,35 @@ __device__ __forceinline__ void conv_span(const ConvParams& p, int total, int nc
                 a[2][e] = xt[e];
             }
         }
-        if (t1 == s1 && p.fin) {
-#pragma unroll
-            for (int e = 0; e < N; ++e) {
-                float* f = p.fin + ((long)s * C + c + e) * 3;
-                f[0] = a[0][e];
-                f[1] = a[1][e];
-                f[2] = a[2][e];
-            }
-        }
+        if (t1 == s1 && p.fin) store_conv_state<N>(p.fin, ((long)s * C + c) * 3, a);
         return;
     }
     // a[j][e]: input at position t - 3 + j of channel c + e (oldest first);
     // before a sequence start the values come from its state, or are zero
     float a[3][N];
-    auto window = [&](int seq, int start, int pos, float (&dst)[N]) {
-        if (pos >= start) {
-            V::load(x + pos * C + c, dst);
-        } else {
-            const int k = 3 + (pos - start);  // 0..2
+    auto window = [&](int seq, int start, int t) {  // before position t of the sequence from `start` on
+        float st[N][3];
+        if (t - 3 < start) {
+            if (p.init) {
+                load_conv_state<N>(p.init, ((long)seq * C + c) * 3, st);
+            } else {
 #pragma unroll
-            for (int e = 0; e < N; ++e) dst[e] = p.init ? p.init[((long)seq * C + c + e) * 3 + k] : 0.f;
+                for (int e = 0; e < N; ++e) st[e][0] = st[e][1] = st[e][2] = 0.f;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const int pos = t - 3 + j;
+            if (pos >= start) {
+                V::load(x + pos * C + c, a[j]);
+            } else {
+                const int k = 3 + (pos - start);  // 0..2
+#pragma unroll
+                for (int e = 0; e < N; ++e) a[j][e] = k == 0 ? st[e][0] : k == 1 ? st[e][1] : st[e][2];
+            }
         }
     };
-#pragma unroll
-    for (int j = 0; j < 3; ++j) window(s, s0, t0 - 3 + j, a[j]);
+    window(s, s0, t0);
     // every input of the span first, so that its loads overlap
     typename V::Raw xs[SPAN];
 #pragma unroll
@@ -218,8 +267,14 @@ __device__ __forceinline__ void conv_span(const ConvParams& p, int total, int nc
             ++s;
             s0 = seq_start(p, s);
             s1 = seq_end(p, s);
+            if constexpr (N == 8) {
+                window(s, s0, s0);
+            } else {  // fp32: the 16-byte form here takes the kernel from 109 to 216 VGPRs
 #pragma unroll
-            for (int j = 0; j < 3; ++j) window(s, s0, s0 - 3 + j, a[j]);
+                for (int j = 0; j < 3; ++j)
+#pragma unroll
+                    for (int e = 0; e < N; ++e) a[j][e] = p.init ? p.init[((long)s * C + c + e) * 3 + j] : 0.f;
+            }
         }
         float xt[N], yt[N];
         V::unpack(xs[i], xt);
@@ -233,24 +288,16 @@ __device__ __forceinline__ void conv_span(const ConvParams& p, int total, int nc
             a[1][e] = a[2][e];
             a[2][e] = xt[e];
         }
-        if (t == s1 - 1 && p.fin) {
-#pragma unroll
-            for (int e = 0; e < N; ++e) {
-                float* f = p.fin + ((long)s * C + c + e) * 3;
-                f[0] = a[0][e];
-                f[1] = a[1][e];
-                f[2] = a[2][e];
-            }
-        }
+        if (t == s1 - 1 && p.fin) store_conv_state<N>(p.fin, ((long)s * C + c) * 3, a);
     }
 }
 
 template <typename T, bool VEC>
-__global__ __launch_bounds__(256) void conv1d_kernel(ConvParams p, int total, int ncb) {
+__global__ __launch_bounds__(256) void conv1d_kernel(ConvParams p, int total, int ncb, int span) {
     using V = Vec<T, VEC>;
     T* __restrict__ y = static_cast<T*>(p.y);
     const long C = p.C;
-    conv_span<T, VEC, kConvSpan>(p, total, ncb, [&](int t, int c, const float (&yt)[V::N]) {
+    conv_span<T, VEC, kConvSpan>(p, total, ncb, span, [&](int t, int c, const float (&yt)[V::N]) {
         V::template store<kConvNT>(y + t * C + c, yt);
     });
 }
@@ -294,7 +341,8 @@ __device__ __forceinline__ float row_sum(float x) {
 }
 
 template <typename T, int G>
-__global__ __launch_bounds__(256, kConvPrepWaves) void conv_prepare_kernel(ConvPrepParams p, int total, int ncb) {
+__global__ __launch_bounds__(256, kConvPrepWaves) void conv_prepare_kernel(ConvPrepParams p, int total, int ncb,
+                                                                          int span) {
     using V = Vec<T, true>;
     constexpr int N = V::N;
     const int H = p.heads, dk = p.d_k, dv = p.d_v;
@@ -302,7 +350,7 @@ __global__ __launch_bounds__(256, kConvPrepWaves) void conv_prepare_kernel(ConvP
     T* __restrict__ qo = static_cast<T*>(p.q);
     T* __restrict__ ko = static_cast<T*>(p.k);
     T* __restrict__ vo = static_cast<T*>(p.v);
-    conv_span<T, true, kConvPrepSpan>(p.conv, total, ncb, [&](int t, int c, const float (&yt)[N]) {
+    conv_span<T, true, kConvPrepSpan>(p.conv, total, ncb, span, [&](int t, int c, const float (&yt)[N]) {
         if (c >= 2 * qk) {  // v (uniform over the row's lanes)
             V::template store<kConvNT>(vo + (long)t * H * dv + (c - 2 * qk), yt);
             return;
@@ -324,10 +372,10 @@ __global__ __launch_bounds__(256, kConvPrepWaves) void conv_prepare_kernel(ConvP
     // The gates of the block's (token, head) pairs, one pair per thread: the
     // blocks holding q channels cover every head once per span.
     const int cb = (blockIdx.x % ncb) * 256 * N;  // first channel of the block
-    const int t0 = (blockIdx.x / ncb) * kConvPrepSpan;
+    const int t0 = (blockIdx.x / ncb) * span;
     if (cb >= qk || t0 >= total) return;
     const int h0 = cb / dk, nh = (min(cb + 256 * N, qk) - cb) / dk;
-    const int nt = min(t0 + kConvPrepSpan, total) - t0;
+    const int nt = min(t0 + span, total) - t0;
     for (int i = threadIdx.x; i < nt * nh; i += 256) {
         const int h = h0 + i % nh;
         const long r = (long)(t0 + i / nh) * H + h;
@@ -535,6 +583,21 @@ hipError_t pick_rows(const P& p, int rows, int n, bool vec, hipStream_t st) {
 
 }  // namespace
 
+// Tokens per span: dense sequences shorter than a span get spans of their own
+// length, so that a block meets one sequence and its one carried state
+// instead of up to `most` of them one after the other: conv_prepare on 64
+// sequences of one token, 6144 bf16 channels, 62 us in spans of 16 tokens
+// (every carried state another round trip of scalar accesses), 32 us with the
+// states read 16 bytes at a time, below the call's 17.6 us on the host in
+// spans of one token; conv1d 60.5 against 10.6 us.
+static int conv_span_len(const int32_t* cu, int seq_len, int most) {
+    return !cu && seq_len > 0 && seq_len < most ? seq_len : most;
+}
+
+// Whether a batch can hold empty sequences (their final state is written by
+// a kernel of its own).
+static bool may_be_empty(const int32_t* cu, int seq_len) { return cu || seq_len == 0; }
+
 hipError_t launch_conv1d(const rhz_conv1d_args& a, hipStream_t st) {
     ConvParams p{a.x, a.weight, a.bias, a.cu_seqlens, a.initial_state, a.final_state, a.y,
                  a.batch, a.seq_len, a.channels};
@@ -544,18 +607,19 @@ hipError_t launch_conv1d(const rhz_conv1d_args& a, hipStream_t st) {
     const int per_thread = vec ? nvec : 1;
     const int ncb = (a.channels / per_thread + 255) / 256;
     if (total > 0) {
-        const dim3 grid((unsigned)((long)ncb * ((total + kConvSpan - 1) / kConvSpan)));
+        const int span = conv_span_len(a.cu_seqlens, a.seq_len, kConvSpan);
+        const dim3 grid((unsigned)((long)ncb * ((total + span - 1) / span)));
         if (a.dtype == RHZ_F32) {
-            if (vec) hipLaunchKernelGGL((conv1d_kernel<float, true>), grid, dim3(256), 0, st, p, total, ncb);
-            else hipLaunchKernelGGL((conv1d_kernel<float, false>), grid, dim3(256), 0, st, p, total, ncb);
+            if (vec) hipLaunchKernelGGL((conv1d_kernel<float, true>), grid, dim3(256), 0, st, p, total, ncb, span);
+            else hipLaunchKernelGGL((conv1d_kernel<float, false>), grid, dim3(256), 0, st, p, total, ncb, span);
         } else {
-            if (vec) hipLaunchKernelGGL((conv1d_kernel<uint16_t, true>), grid, dim3(256), 0, st, p, total, ncb);
-            else hipLaunchKernelGGL((conv1d_kernel<uint16_t, false>), grid, dim3(256), 0, st, p, total, ncb);
+            if (vec) hipLaunchKernelGGL((conv1d_kernel<uint16_t, true>), grid, dim3(256), 0, st, p, total, ncb, span);
+            else hipLaunchKernelGGL((conv1d_kernel<uint16_t, false>), grid, dim3(256), 0, st, p, total, ncb, span);
         }
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    if (a.final_state) {
+    if (a.final_state && may_be_empty(a.cu_seqlens, a.seq_len)) {
         // one channel per thread, whatever the main kernel's vector width
         const int ecb = (a.channels + 255) / 256;
         hipLaunchKernelGGL(conv1d_empty_kernel, dim3(ecb, min(a.batch, 65535)), dim3(256), 0, st, p);
@@ -582,8 +646,9 @@ hipError_t launch_conv_prepare(const rhz_gdr_conv_prepare_args& a, hipStream_t s
     const int g = a.d_k / n;
     const int ncb = (C / n + 255) / 256;
     if (total > 0) {
-        const dim3 grid((unsigned)((long)ncb * ((total + kConvPrepSpan - 1) / kConvPrepSpan)));
-#define RHZ_CONV_PREP(T, G) hipLaunchKernelGGL((conv_prepare_kernel<T, G>), grid, dim3(256), 0, st, p, total, ncb)
+        const int span = conv_span_len(a.cu_seqlens, a.seq_len, kConvPrepSpan);
+        const dim3 grid((unsigned)((long)ncb * ((total + span - 1) / span)));
+#define RHZ_CONV_PREP(T, G) hipLaunchKernelGGL((conv_prepare_kernel<T, G>), grid, dim3(256), 0, st, p, total, ncb, span)
         if (a.dtype == RHZ_F32) {
             switch (g) {
                 case 1: RHZ_CONV_PREP(float, 1); break;
@@ -609,7 +674,7 @@ hipError_t launch_conv_prepare(const rhz_gdr_conv_prepare_args& a, hipStream_t s
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    if (a.final_state) {
+    if (a.final_state && may_be_empty(a.cu_seqlens, a.seq_len)) {
         const int ecb = (C + 255) / 256;
         hipLaunchKernelGGL(conv1d_empty_kernel, dim3(ecb, min(a.batch, 65535)), dim3(256), 0, st, p.conv);
         return hipGetLastError();

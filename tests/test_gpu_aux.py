@@ -467,3 +467,53 @@ def test_local_prefill_empty_sequences_copy_the_state(device):
     _abi.check(_abi.lib().rhz_gdr_local_prefill(byref(la), None))
     torch.cuda.synchronize()
     assert torch.equal(fin, init)
+
+
+@pytest.mark.parametrize("dtype,tol", PATHS)
+@pytest.mark.parametrize("B,T", [(5, 1), (1, 1), (3, 2), (4, 15), (2, 16), (3, 17), (40, 3)])
+@pytest.mark.parametrize("state", ["none", "aligned", "off by one float", "in place"])
+def test_conv_short_sequences(device, dtype, tol, B, T, state):
+    """Dense sequences around one span of 16 tokens (shorter ones get spans of
+    their own length), with the carried state absent, read and written by
+    16-byte accesses, off 16-byte alignment, and updated in place -- against
+    f64, with the final states exact; and the same batch packed."""
+    H, d = 3, 64
+    C = 3 * H * d
+    gen = torch.Generator(device=device).manual_seed(100 * B + T)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=device)  # noqa: E731
+    x, w, bias, a = rand(B, T, C).to(dtype), rand(C, 4), rand(C), rand(H)
+    lg = rand(B, T, H)
+    init = None
+    if state != "none":
+        buf = rand(B * C * 3 + 1)
+        init = buf[1:].view(B, C, 3) if state == "off by one float" else buf[:-1].view(B, C, 3)
+    past = torch.zeros(B, 3, C, device=device) if init is None else init.transpose(1, 2)
+    xx = torch.cat([past.double(), x.double()], 1)
+    y = bias.double() + sum(w[:, j].double() * xx[:, j:j + T] for j in range(4))
+    fin_ref = xx[:, T:].transpose(1, 2).float()
+    host = lambda t: t.float().cpu().numpy()  # noqa: E731
+    cu = torch.arange(0, B * T + 1, T, dtype=torch.int32, device=device)
+    for packed in (False, True):
+        xs, cus = (x.view(B * T, C), cu) if packed else (x, None)
+        out, fin = rhizome_amd.causal_conv1d(xs, w, bias, cu_seqlens=cus, initial_state=init,
+                                             output_final_state=True)
+        check_close(host(out).reshape(B, T, C), y.cpu().numpy(), tol, f"conv1d packed={packed}")
+        assert torch.equal(fin, fin_ref)
+    if state == "in place" and T < 16:  # one block holds a sequence's channels: read, then written
+        import ctypes
+
+        from rhizome_amd import _abi
+
+        st, yy = init.clone(), torch.empty_like(x)
+        args = _abi.Conv1dArgs(B, T, C, _abi.BF16 if dtype == torch.bfloat16 else _abi.F32, x.data_ptr(), w.data_ptr(),
+                               bias.data_ptr(), None, st.data_ptr(), st.data_ptr(), yy.data_ptr())
+        _abi.check(_abi.lib().rhz_causal_conv1d(ctypes.byref(args), torch.cuda.current_stream().cuda_stream or None))
+        check_close(host(yy), y.cpu().numpy(), tol, "conv1d in place")
+        assert torch.equal(st, fin_ref)
+    q, k, v, beta, g, fin = rhizome_amd.conv_prepare(x, w, bias, lg, lg, a, heads=H, d_k=d, d_v=d, initial_state=init,
+                                                     output_final_state=True)
+    yq, yk, yv = (y[..., i * H * d:(i + 1) * H * d].reshape(B, T, H, d) for i in range(3))
+    unit = lambda t: t / t.norm(dim=-1, keepdim=True)  # noqa: E731
+    for got, ref in ((q, unit(yq) * d ** 0.5), (k, unit(yk)), (v, yv), (beta, torch.sigmoid(lg.double()))):
+        check_close(host(got), ref.cpu().numpy(), tol, "conv_prepare")
+    assert torch.equal(fin, fin_ref)
