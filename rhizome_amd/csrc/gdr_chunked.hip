@@ -102,6 +102,10 @@ struct ChunkParams {
 hipError_t chunked_go_prologue(const ChunkParams& cp, int dk, int blocks, hipStream_t st);
 // which: 0 = LDS waits that gave up, 1 = fp16 range errors, 2 = exact reruns.
 hipError_t chunked_prologue_counter(int which, unsigned int* count, bool reset);
+// The same of the narrow instances (gdr_chunked_narrow.hip), kept apart for
+// the same reason.
+hipError_t chunked_go_narrow(const ChunkParams& cp, int dk, int blocks, hipStream_t st);
+hipError_t chunked_narrow_counter(int which, unsigned int* count, bool reset);
 
 namespace {
 
@@ -124,6 +128,8 @@ __device__ unsigned int g_range_errors;
 __device__ unsigned int g_exact_reruns;
 
 constexpr int kTV = 32;           // rows of S per workgroup (two scan waves of 16)
+constexpr int kTVNarrow = 16;     // the same in the narrow instances (one scan wave)
+constexpr int kCUs = 256;
 constexpr int kMaxSortSeqs = 4096;
 constexpr int kMaxScaleExp = 60;  // bound on one rescaling step
 constexpr int kMaxStateExp = 96;  // bound on the state exponent F
@@ -346,7 +352,7 @@ __device__ __forceinline__ int rescale_shift_lanes(float loc, int F) {
 }
 
 // ------------------------------------------------------------ varlen setup
-#ifndef RHZ_CHUNKED_PROLOGUE_TU  // launched by the plain unit's host code only
+#if !defined(RHZ_CHUNKED_PROLOGUE_TU) && !defined(RHZ_CHUNKED_NARROW_TU)  // launched by the plain unit's host code only
 // Longest-first order of the packed sequences (ties by index), so the
 // longest chunk loops start first.  Identity above kMaxSortSeqs sequences.
 __global__ __launch_bounds__(1024) void gdr_varlen_order_kernel(const int* cu, int n, int seq_len, int* order) {
@@ -394,10 +400,10 @@ struct Sync {
     int staged;  // loader waves (4 per chunk): K, Q, beta V, gates in LDS
     int tdiag;   // wave 2 (1 per chunk): K K^T diagonal blocks and T's diagonal blocks
     int aoff;    // wave 3 (1 per chunk): A below the diagonal
-    int tfull;   // waves 2, 3 (2 per chunk): T complete
-    int pdone;   // loader waves 0-2 (3 per chunk): P's first three block rows
+    int tfull;   // waves 2, 3 (2 per chunk): T complete (and, before it, the waves' blocks of P)
+    int pdone;   // loader waves 0-2 (3 per chunk; narrow: 1 and 2, 2 per chunk): P's first three block rows
     int pdone3;  // wave 3 (1 per chunk): P's last block row
-    int scanned[2];  // scan wave w (1 per chunk): its last read of the chunk's buffers returned
+    int scanned[2];  // scan wave w (1 per chunk): its last read of the chunk's buffers returned (narrow: wave 0 only)
     int rerun;       // nonzero: an input left the fp16 path's domain (set once, read after the loops)
 };
 
@@ -530,6 +536,7 @@ struct ChunkIn {
 template <int DK>
 struct LoadOffsets {
     uint32_t kq[DK / 32], v, g, bv;
+    template <bool NARROW>
     __device__ __forceinline__ void set(const ChunkParams& p, int i0, int lt, int last) {
         constexpr int PPR = DK / 8;
         const uint32_t H = p.heads, dk = p.d_k, dv = p.d_v;
@@ -539,7 +546,9 @@ struct LoadOffsets {
             kq[u] = (uint32_t(row) * H * dk + c8) * 2u;
         }
         const int vrow = min(lt >> 2, last);
-        v = (uint32_t(vrow) * H * dv + uint32_t(min(i0 + (lt & 3) * 8, p.d_v - 8) - i0)) * 2u;
+        // (narrow: the lanes of columns 16..31 repeat column 8's piece, whose rows of beta V no wave reads)
+        const int c8 = NARROW ? min((lt & 3) * 8, kTVNarrow - 8) : (lt & 3) * 8;
+        v = (uint32_t(vrow) * H * dv + uint32_t(min(i0 + c8, p.d_v - 8) - i0)) * 2u;
         g = uint32_t(min(lt & 63, last)) * H * 4u;
         bv = uint32_t(vrow) * H * 4u;
     }
@@ -593,8 +602,12 @@ __device__ __forceinline__ void load_chunk_any(const ChunkParams& p, const Unit&
 // exp(G_s) for prod_{u <= s} alpha_u only where seg_s == 0.  Everything from
 // a reset on is then computed from the same numbers whatever came before
 // it.  Tokens past the chunk's end get g = 0 and beta = 0.
-template <int DK, int NB, bool SEG>
-__device__ __forceinline__ void stage_gates_as(Smem<DK>& sm, int s, float g, float beta, bool rst) {
+struct GateVals {
+    float G, gam, gdl, dst, den, pf, beta, sg;
+    bool seg;  // the chunk has a reset (uniform)
+};
+template <bool SEG>
+__device__ __forceinline__ GateVals gate_vals_as(int s, float g, float beta, bool rst) {
     const float sg = SEG ? wave_incl_scan(rst ? 1.f : 0.f) : 0.f;  // small integers: exact
     const float G = SEG ? wave_seg_scan(g, sg) : wave_incl_scan(g);
     const float Glast = lane_val(G, 63);
@@ -624,17 +637,21 @@ __device__ __forceinline__ void stage_gates_as(Smem<DK>& sm, int s, float g, flo
         const float si = bi == 1 ? SB1 : bi == 2 ? SB2 : SB3;
         const float sj = bj == 0 ? SE0 : bj == 1 ? SE1 : SE2;
         pf = si == sj ? pf : 0.f;
-        sm.seg[NB][s] = sg;
     }
-    sm.gcum[NB][s] = G;
-    sm.gam[NB][s] = gam;
-    sm.gdl[NB][s] = gdl;
-    sm.nbg[NB][s] = -beta * gam;
-    sm.bs[NB][s] = beta;
-    sm.dst[NB][s] = dst;
-    sm.den[NB][s] = den;
-    if (s < 16) sm.pf[NB][s] = pf;
-    if (s == 0) sm.resets[NB] = SEG;
+    return {G, gam, gdl, dst, den, pf, beta, sg, SEG};
+}
+template <int DK, int NB>
+__device__ __forceinline__ void write_gates(Smem<DK>& sm, int s, const GateVals& v) {
+    if (v.seg) sm.seg[NB][s] = v.sg;
+    sm.gcum[NB][s] = v.G;
+    sm.gam[NB][s] = v.gam;
+    sm.gdl[NB][s] = v.gdl;
+    sm.nbg[NB][s] = -v.beta * v.gam;
+    sm.bs[NB][s] = v.beta;
+    sm.dst[NB][s] = v.dst;
+    sm.den[NB][s] = v.den;
+    if (s < 16) sm.pf[NB][s] = v.pf;
+    if (s == 0) sm.resets[NB] = v.seg;
 }
 // PRE: the gate and beta loaded are logits, mapped as the prologue does
 // (g = -softplus(a_h) softplus(alpha_logit), beta = sigmoid(beta_logit)).
@@ -646,9 +663,9 @@ struct GateDomain {
     int nan = 0;
     __device__ __forceinline__ bool bad() const { return nan != 0 || !(gmax <= 0.5f); }
 };
-template <int DK, int NB, bool PRE>
-__device__ __forceinline__ void stage_gates(const ChunkParams& p, Smem<DK>& sm, const Unit& u, int s, int len,
-                                            const ChunkIn<DK>& r, GateDomain& dom) {
+template <int DK, bool PRE>
+__device__ __forceinline__ GateVals gate_vals(const ChunkParams& p, const Unit& u, int s, int len,
+                                              const ChunkIn<DK>& r, GateDomain& dom) {
     const float graw = PRE ? -u.spa * fast_softplus(r.g) : log_decay(r.g, p.gate_is_alpha);
     const bool rst = s < len && is_reset(graw);
     const float g = s < len && !rst ? graw : 0.f;
@@ -657,10 +674,8 @@ __device__ __forceinline__ void stage_gates(const ChunkParams& p, Smem<DK>& sm, 
         dom.gmax = fmaxf(dom.gmax, fmaxf(graw + 0.5f, fabsf(beta - 0.5f)));
         dom.nan |= __builtin_isunordered(graw, beta) ? 1 : 0;
     }
-    if (__builtin_amdgcn_ballot_w64(rst) == 0)
-        stage_gates_as<DK, NB, false>(sm, s, g, beta, rst);
-    else
-        stage_gates_as<DK, NB, true>(sm, s, g, beta, rst);
+    return __builtin_amdgcn_ballot_w64(rst) == 0 ? gate_vals_as<false>(s, g, beta, rst)
+                                                 : gate_vals_as<true>(s, g, beta, rst);
 }
 
 // Chunk inputs from registers into LDS buffer NB: K and Q as fp16, beta V
@@ -699,7 +714,7 @@ __device__ __forceinline__ void stage_chunk(const ChunkParams& p, Smem<DK>& sm, 
             sm.vb[NB][(c8 + 2 * e) * kLDV + row] = ok ? bv * __uint_as_float(wv[e] << 16) : 0.f;
             sm.vb[NB][(c8 + 2 * e + 1) * kLDV + row] = ok ? bv * __uint_as_float(wv[e] & 0xffff0000u) : 0.f;
         }
-        if constexpr (GATES) stage_gates<DK, NB, true>(p, sm, un, lt & 63, len, r, dom);
+        if constexpr (GATES) write_gates<DK, NB>(sm, lt & 63, gate_vals<DK, true>(p, un, lt & 63, len, r, dom));
         return;
     }
     const bool full = len == kChunk && p.d_k == DK && i0 + kTV <= p.d_v;  // uniform
@@ -748,7 +763,72 @@ __device__ __forceinline__ void stage_chunk(const ChunkParams& p, Smem<DK>& sm, 
             sm.vb[NB][(c8 + 2 * e + 1) * kLDV + row] = ok ? r.bv * __uint_as_float(wv[e] & 0xffff0000u) : 0.f;
         }
     }
-    if constexpr (GATES) stage_gates<DK, NB, false>(p, sm, un, lt & 63, len, r, dom);
+    if constexpr (GATES) write_gates<DK, NB>(sm, lt & 63, gate_vals<DK, false>(p, un, lt & 63, len, r, dom));
+}
+
+// The narrow instances' staging in two steps, so that only the LDS writes
+// wait for the buffer: their chunk period is the loop from the scan's release
+// of a buffer over its staging, T's blocks and the scan's second half.
+// prepare: K and Q to fp16 in place, beta V as the pairs its 8-byte writes
+// take (as in stage_chunk), and (GATES) the chunk's decay vectors.
+template <int DK>
+struct Prepared {
+    float2 pair[4];
+    GateVals gates;
+};
+template <int DK, bool GATES>
+__device__ __forceinline__ Prepared<DK> prepare_chunk(const ChunkParams& p, const Unit& un, int len, int lt,
+                                                      ChunkIn<DK>& r, GateDomain& dom) {
+    constexpr int PPR = DK / 8;
+    const bool full = len == kChunk && p.d_k == DK && un.i0 + kTVNarrow <= p.d_v;  // uniform
+    Prepared<DK> pr;
+    if (!full) {
+        const uint4 z = make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < DK / 32; ++u) {
+            const int it = lt + 256 * u;
+            const bool ok = it / PPR < len && (it % PPR) * 8 < p.d_k;
+            if (!ok) r.k[u] = r.q[u] = z;
+        }
+        if (!((lt >> 2) < len && un.i0 + (lt & 3) * 8 < p.d_v)) r.v = z, r.bv = 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < DK / 32; ++u) {
+        r.k[u] = bf16x8_to_f16x8(r.k[u]);
+        r.q[u] = bf16x8_to_f16x8(r.q[u]);
+    }
+    const bool odd = (lt >> 2) & 1;
+    const uint32_t wv[4] = {r.v.x, r.v.y, r.v.z, r.v.w};
+    float val[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        val[2 * e] = r.bv * __uint_as_float(wv[e] << 16);
+        val[2 * e + 1] = r.bv * __uint_as_float(wv[e] & 0xffff0000u);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        // lane ^ 4: row_half_mirror, then quad_perm [3, 2, 1, 0]
+        const float recv = dpp_mov<0x1B>(dpp_mov<0x141>(odd ? val[k] : val[4 + k]));
+        pr.pair[k] = odd ? make_float2(recv, val[4 + k]) : make_float2(val[k], recv);
+    }
+    if constexpr (GATES) pr.gates = gate_vals<DK, false>(p, un, lt & 63, len, r, dom);
+    return pr;
+}
+template <int DK, int NB, bool GATES>
+__device__ __forceinline__ void write_chunk(Smem<DK>& sm, int lt, const ChunkIn<DK>& r, const Prepared<DK>& pr) {
+    constexpr int PPR = DK / 8;
+    if constexpr (GATES) write_gates<DK, NB>(sm, lt & 63, pr.gates);
+#pragma unroll
+    for (int u = 0; u < DK / 32; ++u) {
+        const int it = lt + 256 * u, row = it / PPR, c8 = (it % PPR) * 8;
+        *reinterpret_cast<uint4*>(&sm.k[NB][KQ<DK>::off(row, c8)]) = r.k[u];
+        *reinterpret_cast<uint4*>(&sm.q[NB][KQ<DK>::off(row, c8)]) = r.q[u];
+    }
+    const int row = lt >> 2, c8 = (lt & 3) * 8;
+    const bool odd = row & 1;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        *reinterpret_cast<float2*>(&sm.vb[NB][(c8 + k + (odd ? 4 : 0)) * kLDV + row - (odd ? 1 : 0)]) = pr.pair[k];
 }
 
 // ------------------------------------------------------------ K K^T, Q K^T
@@ -907,15 +987,19 @@ template <int DK, int NB>
 __device__ __forceinline__ void qk_blocks_w3(Smem<DK>& sm, int l, uint32_t& rng, const f16x8 (&kr)[4][DK / 32]);
 
 // ------------------------------------------------------------ prep roles
-// Wave 2, chunk x (buffer B = x & 1): K K^T's diagonal blocks and T's
-// diagonal blocks, then T_10, T_20, T_30.
-template <int DK, int B>
-__device__ __forceinline__ void prep_wave2(Smem<DK>& sm, int x, int l, int lim, float& kmax) {
+// Chunk x (buffer B = x & 1): K K^T's diagonal blocks and T's diagonal
+// blocks (wave 2; wave 1 of the narrow instances).
+template <int DK, int B, bool NARROW>
+__device__ __forceinline__ void prep_diag(Smem<DK>& sm, int x, int l, int lim, float& kmax) {
     constexpr int NK = DK / 32;
     const int n = l & 15, g = l >> 4;
     // K[B] staged; T[B] was read by the scan and written by both waves for chunk x - 2
     Sync& sy = sm.sync;
-    wait_all<4>(lim, {&sy.staged, &sy.scanned[0], &sy.scanned[1], &sy.tfull}, {4 * (x + 1), x - 1, x - 1, 2 * (x - 1)});
+    if constexpr (NARROW)
+        wait_all<3>(lim, {&sy.staged, &sy.scanned[0], &sy.tfull}, {4 * (x + 1), x - 1, 2 * (x - 1)});
+    else
+        wait_all<4>(lim, {&sy.staged, &sy.scanned[0], &sy.scanned[1], &sy.tfull},
+                    {4 * (x + 1), x - 1, x - 1, 2 * (x - 1)});
     f16x8 kr[4][NK];
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) load_rows<DK>(sm.k[B], blk, n, g, kr[blk]);
@@ -937,13 +1021,36 @@ __device__ __forceinline__ void prep_wave2(Smem<DK>& sm, int x, int l, int lim, 
     lds_fence();
     t_diag<DK, B>(sm, l);
     signal(&sm.sync.tdiag);
-    wait_ge(lim, &sm.sync.aoff, x + 1);
+}
+
+// T_10, T_20, T_30 of buffer B, its diagonal blocks and A's blocks there.
+template <int DK, int B>
+__device__ __forceinline__ void t_column0(Smem<DK>& sm, int l) {
     t_block<DK, B, 1, 0>(sm, l);
     lds_fence();
     t_block<DK, B, 2, 0>(sm, l);
     lds_fence();
     t_block<DK, B, 3, 0>(sm, l);
     signal(&sm.sync.tfull);
+}
+
+// Wave 2, chunk x: the diagonal blocks, then T_10, T_20, T_30.
+template <int DK, int B>
+__device__ __forceinline__ void prep_wave2(Smem<DK>& sm, int x, int l, int lim, float& kmax) {
+    prep_diag<DK, B, false>(sm, x, l, lim, kmax);
+    wait_ge(lim, &sm.sync.aoff, x + 1);
+    t_column0<DK, B>(sm, l);
+}
+
+// Wave 2 of the narrow instances, chunk x: Q K^T's blocks (0,0) and (1,0),
+// then T_10, T_20, T_30 once wave 1 has the diagonal blocks.  P[B] and T[B]
+// were read by the scan for chunk x - 2 before x was staged.
+template <int DK, int B>
+__device__ __forceinline__ void prep_column0(Smem<DK>& sm, int x, int l, int lim, uint32_t& rng) {
+    wait_ge(lim, &sm.sync.staged, 4 * (x + 1));
+    qk_blocks<DK, B, 0>(sm, l, rng);  // counted with T's blocks in tfull
+    wait_all<2>(lim, {&sm.sync.tdiag, &sm.sync.aoff}, {x + 1, x + 1});
+    t_column0<DK, B>(sm, l);
 }
 
 // Wave 3, chunk x: K K^T below the diagonal into A, then T_32, T_21, T_31.
@@ -1064,42 +1171,51 @@ __device__ __forceinline__ void qk_blocks_w3(Smem<DK>& sm, int l, uint32_t& rng,
 // Loader wave LW, chunk x (buffer B = x & 1): stage x from registers, load
 // x + 2 into the same registers, then Q K^T of x.  Each register set has
 // two chunk periods to arrive.
-template <int DK, int B, int LW, bool PRE>
+template <int DK, int B, int LW, bool PRE, bool NARROW>
 __device__ __forceinline__ void prep_loader(const ChunkParams& p, Smem<DK>& sm, const Unit& u, int x, int lt,
                                             const LoadOffsets<DK>& lo, const LoadOffsets<DK>& lastc,
                                             ChunkIn<DK>& in, uint32_t& rng, GateDomain& dom) {
     // buffer B held chunk x - 2: every reader of it is done (nothing to wait for when x < 2)
     Sync& sy = sm.sync;
-    wait_all<6>(p.spin_limit, {&sy.scanned[0], &sy.scanned[1], &sy.pdone, &sy.pdone3, &sy.tdiag, &sy.aoff},
-                {x - 1, x - 1, 3 * (x - 1), x - 1, x - 1, x - 1});
     const int len = min(kChunk, u.te - (u.tb + x * kChunk));
-    stage_chunk<DK, B, LW == kGateWave, PRE>(p, sm, u, len, u.i0, lt, in, dom);
+    if constexpr (NARROW) {
+        static_assert(!PRE, "the fused prologue has no narrow instances");
+        const Prepared<DK> pr = prepare_chunk<DK, LW == kGateWave>(p, u, len, lt, in, dom);
+        wait_all<5>(p.spin_limit, {&sy.scanned[0], &sy.pdone, &sy.pdone3, &sy.tdiag, &sy.aoff},
+                    {x - 1, 2 * (x - 1), x - 1, x - 1, x - 1});
+        write_chunk<DK, B, LW == kGateWave>(sm, lt, in, pr);
+    } else {
+        wait_all<6>(p.spin_limit, {&sy.scanned[0], &sy.scanned[1], &sy.pdone, &sy.pdone3, &sy.tdiag, &sy.aoff},
+                    {x - 1, x - 1, 3 * (x - 1), x - 1, x - 1, x - 1});
+        stage_chunk<DK, B, LW == kGateWave, PRE>(p, sm, u, len, u.i0, lt, in, dom);
+    }
     signal(&sm.sync.staged);
     load_chunk_any<DK>(p, u, x + 2, lo, lastc, in);
     // every loader waits for all four to have staged x, so that none stages
     // x + 1 first (staged counts 4 per chunk)
     wait_ge(p.spin_limit, &sm.sync.staged, 4 * (x + 1));
-    if constexpr (LW != kGateWave) {  // the gate loader's Q K^T blocks are wave 3's
+    // the gate loader's Q K^T blocks are wave 3's, the narrow instances' loader 0's are wave 2's
+    if constexpr (LW != kGateWave && !(NARROW && LW == 0)) {
         qk_blocks<DK, B, LW>(sm, lt & 63, rng);
         signal(&sm.sync.pdone);
     }
 }
 
-template <int DK, int LW, bool PRE>
+template <int DK, int LW, bool PRE, bool NARROW>
 __device__ __forceinline__ void loader_loop(const ChunkParams& p, Smem<DK>& sm, const Unit& u, int lt) {
     if (u.nch <= 0) return;
     LoadOffsets<DK> lo, lastc;
-    lo.set(p, u.i0, lt, kChunk - 1);
-    lastc.set(p, u.i0, lt, u.te - (u.tb + (u.nch - 1) * kChunk) - 1);
+    lo.template set<NARROW>(p, u.i0, lt, kChunk - 1);
+    lastc.template set<NARROW>(p, u.i0, lt, u.te - (u.tb + (u.nch - 1) * kChunk) - 1);
     ChunkIn<DK> in0, in1;
     load_chunk_any<DK>(p, u, 0, lo, lastc, in0);
     load_chunk_any<DK>(p, u, 1, lo, lastc, in1);
     uint32_t rng = 0;
     GateDomain dom;
     for (int x = 0; x < u.nch; x += 2) {
-        prep_loader<DK, 0, LW, PRE>(p, sm, u, x, lt, lo, lastc, in0, rng, dom);
+        prep_loader<DK, 0, LW, PRE, NARROW>(p, sm, u, x, lt, lo, lastc, in0, rng, dom);
         if (x + 1 >= u.nch) break;
-        prep_loader<DK, 1, LW, PRE>(p, sm, u, x + 1, lt, lo, lastc, in1, rng, dom);
+        prep_loader<DK, 1, LW, PRE, NARROW>(p, sm, u, x + 1, lt, lo, lastc, in1, rng, dom);
     }
     if constexpr (PRE)
         note_range(rng);
@@ -1126,7 +1242,7 @@ __device__ __forceinline__ float state_max(const ScanState<DK>& st) {
 }
 
 // Chunk c of a scan wave (w = 0, 1) on buffer B = c & 1.
-template <int DK, int B>
+template <int DK, int B, bool NARROW>
 __device__ __forceinline__ void scan_chunk(const ChunkParams& p, Smem<DK>& sm, const Unit& u, int c, int w, int l,
                                            ScanState<DK>& st) {
     constexpr int NK = DK / 32;  // 32-wide contraction steps over d_k
@@ -1233,7 +1349,12 @@ __device__ __forceinline__ void scan_chunk(const ChunkParams& p, Smem<DK>& sm, c
         for (int tb2 = 0; tb2 < 4; ++tb2) OQ[tb2] *= gq[tb2] * fo;
     }
     // ---- U = T Rhat, O^T += U^T P^T, S update.
-    wait_all<3>(p.spin_limit, {&sm.sync.tfull, &sm.sync.pdone, &sm.sync.pdone3}, {2 * (c + 1), 3 * (c + 1), c + 1});
+    if constexpr (NARROW)
+        wait_all<3>(p.spin_limit, {&sm.sync.tfull, &sm.sync.pdone, &sm.sync.pdone3},
+                    {2 * (c + 1), 2 * (c + 1), c + 1});
+    else
+        wait_all<3>(p.spin_limit, {&sm.sync.tfull, &sm.sync.pdone, &sm.sync.pdone3},
+                    {2 * (c + 1), 3 * (c + 1), c + 1});
     {
         const int F1 = st.F + er;
         // T rows (both 32-token halves for rows >= 32), P rows, decays.
@@ -1332,15 +1453,17 @@ __device__ __forceinline__ void scan_chunk(const ChunkParams& p, Smem<DK>& sm, c
 
 // ------------------------------------------------------------ fused kernel
 // Shared memory of the chunk loops, reused by the exact rerun.
-template <int DK>
+template <int DK, bool NARROW>
 union KernelSmem {
+    // waves of the exact rerun: 8 rows each, one tile
+    static constexpr int RW = (NARROW ? kTVNarrow : kTV) / 8;
     Smem<DK> chunk;
-    StageSmem<8> rerun;  // 16 * 8 = 128 key columns, 32 rows: one tile
+    StageSmem<8, 16, RW> rerun;  // 16 * 8 = 128 key columns
+    static_assert(StageSmem<8, 16, RW>::RPB == 8 * RW, "the exact rerun covers one tile of rows");
 };
-static_assert(StageSmem<8>::RPB == kTV, "the exact rerun covers one tile of rows");
 
 // Workgroup bid -> its (sequence, head, rows) and token range.
-template <bool PRE>
+template <bool PRE, bool NARROW>
 __device__ __forceinline__ Unit make_unit(const ChunkParams& p, int bid) {
     const int H = p.heads;
     int unit, tile;
@@ -1353,7 +1476,7 @@ __device__ __forceinline__ Unit make_unit(const ChunkParams& p, int bid) {
     u.seq = p.order ? min(max(p.order[seqi], 0), p.batch - 1) : seqi;
     seq_bounds(p.cu_seqlens, u.seq, p.seq_len, u.tb, u.te);
     u.nch = (u.te - u.tb + kChunk - 1) / kChunk;
-    u.i0 = tile * kTV;
+    u.i0 = tile * (NARROW ? kTVNarrow : kTV);
     u.spa = PRE && u.nch > 0 ? softplus_f(p.a_log[u.h]) : 0.f;
     return u;
 }
@@ -1363,22 +1486,27 @@ __device__ __forceinline__ Unit make_unit(const ChunkParams& p, int bid) {
 // tile's rows from the initial state with the fp32 recurrence, overwriting
 // the outputs and the final state the chunk loops wrote.  Its arguments
 // come from LDS (rerun_args), read before the rerun reuses that memory.
-template <int DK>
-__device__ __forceinline__ void exact_rerun(KernelSmem<DK>& smu) {
+template <int DK, bool NARROW>
+__device__ __forceinline__ void exact_rerun(KernelSmem<DK, NARROW>& smu) {
     const RerunArgs ra = smu.chunk.rerun_args;
     __syncthreads();  // every wave has read the flag and the arguments: the LDS is free
-    staged_rows<8, uint16_t>(ra.sp, smu.rerun, ra.seq, ra.h, ra.i0, threadIdx.x);
+    staged_rows<8, uint16_t, 16, KernelSmem<DK, NARROW>::RW>(ra.sp, smu.rerun, ra.seq, ra.h, ra.i0, threadIdx.x);
 }
 
 // PRE: the fused prologue (raw q, k projections and gate / beta logits).
-template <int DK, bool PRE>
+// NARROW: 16 rows of S per workgroup, for launches that leave CUs idle (the
+// rule is at the launch).  One wave scans (wave 0); wave 1 takes wave 2's
+// K K^T and substitution, and wave 2 loader 0's Q K^T blocks, so that the
+// scan shares its SIMD only with a loader's staging.  The same numbers are
+// formed from the same operands, so both forms' results are bit-identical.
+template <int DK, bool PRE, bool NARROW>
 __global__ __launch_bounds__(512) void gdr_chunk_kernel(ChunkParams p) {
     constexpr int NK = DK / 32;
-    __shared__ __align__(16) KernelSmem<DK> smu;
+    __shared__ __align__(16) KernelSmem<DK, NARROW> smu;
     Smem<DK>& sm = smu.chunk;
 
     const int H = p.heads;
-    const Unit u = make_unit<PRE>(p, blockIdx.x);
+    const Unit u = make_unit<PRE, NARROW>(p, blockIdx.x);
     const int tid = threadIdx.x, l = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int dk = p.d_k, dv = p.d_v;
@@ -1399,7 +1527,7 @@ __global__ __launch_bounds__(512) void gdr_chunk_kernel(ChunkParams p) {
 
     // Every role runs chunks 0 .. nch-1, unrolled by two so that buffer c & 1
     // is a compile-time constant.
-    if (w < 2) {
+    if (w < (NARROW ? 1 : 2)) {
         const int n = l & 15, g = l >> 4;
         const int i = u.i0 + 16 * w + n;
         const size_t srow = ((size_t(u.seq) * H + u.h) * dv + i) * dk;
@@ -1419,8 +1547,8 @@ __global__ __launch_bounds__(512) void gdr_chunk_kernel(ChunkParams p) {
         st.F = 0;
         st.smax = state_max(st);
         for (int c = 0; c < u.nch; c += 2) {
-            scan_chunk<DK, 0>(p, sm, u, c, w, l, st);
-            if (c + 1 < u.nch) scan_chunk<DK, 1>(p, sm, u, c + 1, w, l, st);
+            scan_chunk<DK, 0, NARROW>(p, sm, u, c, w, l, st);
+            if (c + 1 < u.nch) scan_chunk<DK, 1, NARROW>(p, sm, u, c + 1, w, l, st);
         }
         if (p.fin && i < dv) {
             const float f = exp2i(st.F);
@@ -1434,13 +1562,32 @@ __global__ __launch_bounds__(512) void gdr_chunk_kernel(ChunkParams p) {
                 }
             }
         }
-    } else if (w == 2) {
+    } else if (NARROW && w == 1) {
         float kmax = 0.f;
         for (int x = 0; x < u.nch; x += 2) {
-            prep_wave2<DK, 0>(sm, x, l, p.spin_limit, kmax);
-            if (x + 1 < u.nch) prep_wave2<DK, 1>(sm, x + 1, l, p.spin_limit, kmax);
+            prep_diag<DK, 0, NARROW>(sm, x, l, p.spin_limit, kmax);
+            if (x + 1 < u.nch) prep_diag<DK, 1, NARROW>(sm, x + 1, l, p.spin_limit, kmax);
         }
         if constexpr (!PRE) flag_rerun(sm, !(kmax <= kKeyNormSqMax));
+    } else if (w == 2) {
+        if constexpr (NARROW) {
+            uint32_t rng = 0;
+            for (int x = 0; x < u.nch; x += 2) {
+                prep_column0<DK, 0>(sm, x, l, p.spin_limit, rng);
+                if (x + 1 < u.nch) prep_column0<DK, 1>(sm, x + 1, l, p.spin_limit, rng);
+            }
+            if constexpr (PRE)
+                note_range(rng);
+            else
+                flag_rerun(sm, range_bad(rng));
+        } else {
+            float kmax = 0.f;
+            for (int x = 0; x < u.nch; x += 2) {
+                prep_wave2<DK, 0>(sm, x, l, p.spin_limit, kmax);
+                if (x + 1 < u.nch) prep_wave2<DK, 1>(sm, x + 1, l, p.spin_limit, kmax);
+            }
+            if constexpr (!PRE) flag_rerun(sm, !(kmax <= kKeyNormSqMax));
+        }
     } else if (w == 3) {
         uint32_t rng = 0;
         for (int x = 0; x < u.nch; x += 2) {
@@ -1452,21 +1599,23 @@ __global__ __launch_bounds__(512) void gdr_chunk_kernel(ChunkParams p) {
         else
             flag_rerun(sm, range_bad(rng));
     } else if (w == 4) {
-        loader_loop<DK, 0, PRE>(p, sm, u, tid - 256);
+        loader_loop<DK, 0, PRE, NARROW>(p, sm, u, tid - 256);
     } else if (w == 5) {
-        loader_loop<DK, 1, PRE>(p, sm, u, tid - 256);
+        loader_loop<DK, 1, PRE, NARROW>(p, sm, u, tid - 256);
     } else if (w == 6) {
-        loader_loop<DK, 2, PRE>(p, sm, u, tid - 256);
+        loader_loop<DK, 2, PRE, NARROW>(p, sm, u, tid - 256);
     } else {
-        loader_loop<DK, 3, PRE>(p, sm, u, tid - 256);
+        loader_loop<DK, 3, PRE, NARROW>(p, sm, u, tid - 256);
     }
 
     if constexpr (!PRE) {
         __syncthreads();  // every role has left its loop and set its flag
         const int rerun = __hip_atomic_load(&sm.sync.rerun, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (rerun != 0) {  // uniform over the workgroup
-            if (threadIdx.x == 0) atomicAdd(&g_exact_reruns, 1u);
-            exact_rerun<DK>(smu);
+            // counted per 32 rows in both forms (the tiles of a head see the same
+            // keys and gates, so they rerun together)
+            if (threadIdx.x == 0 && u.i0 % kTV == 0) atomicAdd(&g_exact_reruns, 1u);
+            exact_rerun<DK, NARROW>(smu);
         }
     }
 }
@@ -1497,30 +1646,44 @@ hipError_t read_counter(int which, unsigned int* count, bool reset) {
     return hipMemcpyFromSymbol(count, HIP_SYMBOL(g_counter_read), sizeof(unsigned int), 0, hipMemcpyDeviceToHost);
 }
 
-#ifndef RHZ_CHUNKED_PROLOGUE_TU
+#if defined(RHZ_CHUNKED_PROLOGUE_TU) || defined(RHZ_CHUNKED_NARROW_TU)
+template <bool PRE, bool NARROW>
+hipError_t go_instances(const ChunkParams& cp, int dk, int blocks, hipStream_t st) {
+    if (dk == 32)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(gdr_chunk_kernel<32, PRE, NARROW>), dim3(blocks), dim3(512), 0, st, cp);
+    else if (dk == 64)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(gdr_chunk_kernel<64, PRE, NARROW>), dim3(blocks), dim3(512), 0, st, cp);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(gdr_chunk_kernel<128, PRE, NARROW>), dim3(blocks), dim3(512), 0, st, cp);
+    return hipGetLastError();
+}
+#else
 template <int DK>
-hipError_t chunked_go(const ChunkParams& cp, int blocks, hipStream_t st) {
+hipError_t chunked_go(const ChunkParams& cp, int blocks, bool narrow, hipStream_t st) {
     if (blocks <= 0) return hipGetLastError();
     if (cp.prologue) return chunked_go_prologue(cp, DK, blocks, st);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(gdr_chunk_kernel<DK, false>), dim3(blocks), dim3(512), 0, st, cp);
+    if (narrow) return chunked_go_narrow(cp, DK, blocks, st);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(gdr_chunk_kernel<DK, false, false>), dim3(blocks), dim3(512), 0, st, cp);
     return hipGetLastError();
 }
 #endif
 
 }  // namespace
 
-#ifdef RHZ_CHUNKED_PROLOGUE_TU
+#if defined(RHZ_CHUNKED_PROLOGUE_TU)
 hipError_t chunked_go_prologue(const ChunkParams& cp, int dk, int blocks, hipStream_t st) {
-    if (dk == 32)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(gdr_chunk_kernel<32, true>), dim3(blocks), dim3(512), 0, st, cp);
-    else if (dk == 64)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(gdr_chunk_kernel<64, true>), dim3(blocks), dim3(512), 0, st, cp);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(gdr_chunk_kernel<128, true>), dim3(blocks), dim3(512), 0, st, cp);
-    return hipGetLastError();
+    return go_instances<true, false>(cp, dk, blocks, st);
 }
 
 hipError_t chunked_prologue_counter(int which, unsigned int* count, bool reset) {
+    return read_counter(which, count, reset);
+}
+#elif defined(RHZ_CHUNKED_NARROW_TU)
+hipError_t chunked_go_narrow(const ChunkParams& cp, int dk, int blocks, hipStream_t st) {
+    return go_instances<false, true>(cp, dk, blocks, st);
+}
+
+hipError_t chunked_narrow_counter(int which, unsigned int* count, bool reset) {
     return read_counter(which, count, reset);
 }
 #else
@@ -1532,25 +1695,22 @@ size_t chunked_workspace_bytes(const rhz_gdr_prefill_args& a) {
     return a.cu_seqlens ? ((sizeof(int) * (size_t)a.batch + 255) & ~size_t(255)) : 0;
 }
 
-// Both counters are the sum of this unit's and the fused-prologue unit's.
-hipError_t chunked_sync_timeouts(unsigned int* count, bool reset) {
-    unsigned int a = 0, b = 0;
-    hipError_t e = read_counter(0, &a, reset);
-    if (e == hipSuccess) e = chunked_prologue_counter(0, &b, reset);
-    *count = a + b;
+namespace {
+// A counter of this unit, of the fused-prologue unit and of the narrow unit,
+// summed.
+hipError_t sum_counters(int which, unsigned int* count, bool reset) {
+    unsigned int a = 0, b = 0, c = 0;
+    hipError_t e = read_counter(which, &a, reset);
+    if (e == hipSuccess) e = chunked_prologue_counter(which, &b, reset);
+    if (e == hipSuccess) e = chunked_narrow_counter(which, &c, reset);
+    *count = a + b + c;
     return e;
 }
+}  // namespace
 
-hipError_t chunked_range_errors(unsigned int* count, bool reset) {
-    unsigned int a = 0, b = 0;
-    hipError_t e = read_counter(1, &a, reset);
-    if (e == hipSuccess) e = chunked_prologue_counter(1, &b, reset);
-    *count = a + b;
-    return e;
-}
-
-// Only the plain instances rerun tiles.
-hipError_t chunked_exact_reruns(unsigned int* count, bool reset) { return read_counter(2, count, reset); }
+hipError_t chunked_sync_timeouts(unsigned int* count, bool reset) { return sum_counters(0, count, reset); }
+hipError_t chunked_range_errors(unsigned int* count, bool reset) { return sum_counters(1, count, reset); }
+hipError_t chunked_exact_reruns(unsigned int* count, bool reset) { return sum_counters(2, count, reset); }
 
 namespace {
 
@@ -1628,7 +1788,14 @@ hipError_t launch_chunked_with(const rhz_gdr_prefill_args& a, hipStream_t st, in
     cp.d_k = a.d_k;
     cp.d_v = a.d_v;
     cp.gate_is_alpha = a.gate_kind == RHZ_GATE_ALPHA;
-    cp.n_tiles = (a.d_v + kTV - 1) / kTV;
+    // One workgroup fills a CU's LDS, so a launch of up to 256 (one per CU) is
+    // one round.  Where workgroups of 16 rows still fit one round, their
+    // shorter chunk period counts (B=1 H=16 T=2043 d=128 58.7 -> 55.5 us; B=1
+    // H=2 T=4333 d=32 101.3 -> 82.8 us); beyond it they would take two rounds
+    // where 32 rows take one.
+    const int narrow_tiles = (a.d_v + kTVNarrow - 1) / kTVNarrow;
+    const bool narrow = !pro && (int64_t)a.batch * a.heads * narrow_tiles <= kCUs;
+    cp.n_tiles = narrow ? narrow_tiles : (a.d_v + kTV - 1) / kTV;
     cp.spin_limit = spin_limit > 0 ? spin_limit : kSpinLimit;
     cp.order = nullptr;
     if (a.cu_seqlens) {
@@ -1639,11 +1806,11 @@ hipError_t launch_chunked_with(const rhz_gdr_prefill_args& a, hipStream_t st, in
         cp.order = order_buf;
     }
     const int blocks = a.batch * a.heads * cp.n_tiles;
-    if (a.d_k <= 32) return chunked_go<32>(cp, blocks, st);
-    if (a.d_k <= 64) return chunked_go<64>(cp, blocks, st);
-    return chunked_go<128>(cp, blocks, st);
+    if (a.d_k <= 32) return chunked_go<32>(cp, blocks, narrow, st);
+    if (a.d_k <= 64) return chunked_go<64>(cp, blocks, narrow, st);
+    return chunked_go<128>(cp, blocks, narrow, st);
 }
 }  // namespace
-#endif  // RHZ_CHUNKED_PROLOGUE_TU
+#endif  // the plain instances' unit
 
 }  // namespace rhz

@@ -214,7 +214,7 @@ class ProtocolError(AssertionError):
     pass
 
 
-def simulate(nch, seed, mistake=None):
+def simulate(nch, seed, mistake=None, roles_of=_roles):
     rng = random.Random(seed)
     cnt = dict(staged=0, tdiag=0, aoff=0, tfull=0, pdone=0, pdone3=0, scanned0=0, scanned1=0)
     buf = {}  # (buffer, index) -> chunk whose data it holds
@@ -227,7 +227,7 @@ def simulate(nch, seed, mistake=None):
     def wr(name, idx, x):
         buf[(name, idx)] = x
 
-    roles = _roles(nch, cnt, rd, wr, mistake)
+    roles = roles_of(nch, cnt, rd, wr, mistake)
     pc = {r: 0 for r in roles}  # next step of each role
     inflight = {}               # role -> step started and not ended
     while True:
@@ -268,6 +268,135 @@ def test_planted_mistakes_are_caught(mistake):
     for seed in range(300):
         try:
             simulate(6, seed, mistake)
+        except ProtocolError:
+            caught += 1
+    assert caught > 0, f"the model did not catch the planted mistake {mistake}"
+
+
+# ---- the narrow instances (16 rows per workgroup): one scan wave; wave 1
+# takes wave 2's diagonal blocks; wave 2 takes loader 0's Q K^T blocks and
+# then T's first block column, counted together in tfull; pdone counts
+# loaders 1 and 2.
+def _narrow_roles(nch, cnt, rd, wr, mistake=None):
+    wide = _roles(nch, cnt, rd, wr)
+
+    def read_all(b, x, names):
+        for L in range(4):
+            for nm in names:
+                rd(nm + str(L), b, x)
+
+    def loader(L):
+        steps = []
+        for x in range(nch):
+            b = x & 1
+
+            def w_stage(x=x):
+                return (cnt["scanned0"] >= x - 1
+                        and cnt["pdone"] >= 2 * (x - 1) and cnt["pdone3"] >= x - 1
+                        and cnt["tdiag"] >= x - 1 and cnt["aoff"] >= x - 1)
+
+            def e_stage(x=x, b=b):
+                for nm in ("k", "q", "vb", "g"):
+                    wr(nm + str(L), b, x)
+                cnt["staged"] += 1
+
+            steps.append((w_stage, lambda: None, e_stage))
+            w_qk = lambda x=x: cnt["staged"] >= 4 * (x + 1)  # noqa: E731
+            if L in (0, 3):
+                steps.append((w_qk, lambda: None, lambda: None))
+                continue
+
+            def e_qk(x=x, b=b):
+                read_all(b, x, ("k", "q", "g"))
+                wr("p" + str(L), b, x)
+                cnt["pdone"] += 1
+
+            steps.append((w_qk, lambda x=x, b=b: read_all(b, x, ("k", "q", "g")), e_qk))
+        return steps
+
+    def wave1():
+        steps = []
+        for x in range(nch):
+            b = x & 1
+
+            def w1(x=x):
+                return (cnt["staged"] >= 4 * (x + 1) and cnt["scanned0"] >= x - 1 and cnt["tfull"] >= 2 * (x - 1))
+
+            def e1(x=x, b=b):
+                read_all(b, x, ("k", "g"))
+                wr("tdiag", b, x)
+                cnt["tdiag"] += 1
+
+            steps.append((w1, lambda x=x, b=b: read_all(b, x, ("k", "g")), e1))
+        return steps
+
+    def wave2():
+        steps = []
+        for x in range(nch):
+            b = x & 1
+
+            def e1(x=x, b=b):
+                read_all(b, x, ("k", "q", "g"))
+                wr("p0", b, x)
+
+            steps.append((lambda x=x: cnt["staged"] >= 4 * (x + 1),
+                          lambda x=x, b=b: read_all(b, x, ("k", "q", "g")), e1))
+
+            def w2(x=x):
+                return cnt["aoff"] >= x + 1 and (mistake == "wave2_ignores_tdiag" or cnt["tdiag"] >= x + 1)
+
+            def s2(x=x, b=b):
+                rd("a", 0, x)
+                rd("tdiag", b, x)
+
+            def e2(x=x, b=b):
+                s2(x, b)
+                wr("toff2", b, x)
+                cnt["tfull"] += 1
+
+            steps.append((w2, s2, e2))
+        return steps
+
+    def scan():
+        steps = []
+        for c in range(nch):
+            b = c & 1
+            sA = lambda c=c, b=b: read_all(b, c, ("k", "q", "vb", "g"))  # noqa: E731
+            steps.append((lambda c=c: cnt["staged"] >= 4 * (c + 1), sA, sA))
+
+            def wB(c=c):
+                return (cnt["tfull"] >= 2 * (c + 1) - (mistake == "scan_waits_for_one_t")
+                        and cnt["pdone"] >= 2 * (c + 1) and cnt["pdone3"] >= c + 1)
+
+            def sB(c=c, b=b):
+                for nm in ("tdiag", "toff2", "toff3", "p0", "p1", "p2", "p3"):
+                    rd(nm, b, c)
+                read_all(b, c, ("k", "g"))
+
+            def eB(c=c, b=b):
+                sB(c, b)
+                cnt["scanned0"] += 1
+
+            steps.append((wB, sB, eB))
+        return steps
+
+    roles = {"L%d" % L: loader(L) for L in range(4)}
+    roles.update(w1=wave1(), w2=wave2(), w3=wide["w3"], s0=scan())
+    return roles
+
+
+@pytest.mark.parametrize("nch", range(0, 8))
+def test_narrow_protocol_no_deadlock_no_stale_read(nch):
+    for seed in range(300):
+        simulate(nch, seed, roles_of=_narrow_roles)
+
+
+@pytest.mark.parametrize("mistake", ["wave2_ignores_tdiag", "scan_waits_for_one_t"])
+def test_narrow_planted_mistakes_are_caught(mistake):
+    caught = 0
+    for seed in range(300):
+        try:
+            simulate(6, seed, mistake, roles_of=_narrow_roles)
         except ProtocolError:
             caught += 1
     assert caught > 0, f"the model did not catch the planted mistake {mistake}"
