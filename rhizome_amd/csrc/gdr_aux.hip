@@ -350,6 +350,22 @@ __global__ __launch_bounds__(256, kConvPrepWaves) void conv_prepare_kernel(ConvP
     T* __restrict__ qo = static_cast<T*>(p.q);
     T* __restrict__ ko = static_cast<T*>(p.k);
     T* __restrict__ vo = static_cast<T*>(p.v);
+    // The gates of the block's (token, head) pairs, one pair per thread: the
+    // blocks holding q channels cover every head once per span.  The first
+    // pair's logits (with 16 heads a whole span's) are read ahead of the
+    // convolution, so that their latency does not follow it.
+    const int cb = (blockIdx.x % ncb) * 256 * N;  // first channel of the block
+    const int t0 = (blockIdx.x / ncb) * span;
+    const int h0 = cb / dk, nh = cb < qk ? (min(cb + 256 * N, qk) - cb) / dk : 0;
+    const int pairs = max(min(t0 + span, total) - t0, 0) * nh;
+    float bl = 0.f, al = 0.f, ah = 0.f;
+    if (int(threadIdx.x) < pairs) {
+        const int h = h0 + threadIdx.x % nh;
+        const long r = (long)(t0 + threadIdx.x / nh) * H + h;
+        bl = p.beta_logit[r];
+        al = p.alpha_logit[r];
+        ah = p.a_log[h];
+    }
     conv_span<T, true, kConvPrepSpan>(p.conv, total, ncb, span, [&](int t, int c, const float (&yt)[N]) {
         if (c >= 2 * qk) {  // v (uniform over the row's lanes)
             V::template store<kConvNT>(vo + (long)t * H * dv + (c - 2 * qk), yt);
@@ -369,18 +385,16 @@ __global__ __launch_bounds__(256, kConvPrepWaves) void conv_prepare_kernel(ConvP
         for (int e = 0; e < N; ++e) o[e] = yt[e] * f;
         V::template store<kRowNT>((isq ? qo : ko) + (long)t * qk + cc, o);
     });
-    // The gates of the block's (token, head) pairs, one pair per thread: the
-    // blocks holding q channels cover every head once per span.
-    const int cb = (blockIdx.x % ncb) * 256 * N;  // first channel of the block
-    const int t0 = (blockIdx.x / ncb) * span;
-    if (cb >= qk || t0 >= total) return;
-    const int h0 = cb / dk, nh = (min(cb + 256 * N, qk) - cb) / dk;
-    const int nt = min(t0 + span, total) - t0;
-    for (int i = threadIdx.x; i < nt * nh; i += 256) {
+    for (int i = threadIdx.x; i < pairs; i += 256) {
         const int h = h0 + i % nh;
         const long r = (long)(t0 + i / nh) * H + h;
-        p.beta[r] = sigmoid_f(p.beta_logit[r]);
-        p.g[r] = -softplus_f(p.a_log[h]) * softplus_f(p.alpha_logit[r]);
+        if (i >= 256) {
+            bl = p.beta_logit[r];
+            al = p.alpha_logit[r];
+            ah = p.a_log[h];
+        }
+        p.beta[r] = sigmoid_f(bl);
+        p.g[r] = -softplus_f(ah) * softplus_f(al);
     }
 }
 
