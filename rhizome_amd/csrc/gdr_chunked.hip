@@ -110,7 +110,7 @@ hipError_t chunked_narrow_counter(int which, unsigned int* count, bool reset);
 namespace {
 
 // Number of LDS waits that gave up since the last reset (per device and
-// compilation unit: the host adds the two units' counts).
+// compilation unit: the host adds the units' counts).
 __device__ unsigned int g_sync_timeouts;
 // Number of (workgroup, wave) pairs since the last reset in which an fp16
 // entry of A or P (the MFMA operands formed from q and k) was NaN,
