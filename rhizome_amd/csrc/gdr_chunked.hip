@@ -1493,6 +1493,11 @@ __device__ __forceinline__ void exact_rerun(KernelSmem<DK, NARROW>& smu) {
     staged_rows<8, uint16_t, 16, KernelSmem<DK, NARROW>::RW>(ra.sp, smu.rerun, ra.seq, ra.h, ra.i0, threadIdx.x);
 }
 
+template <int DK>
+__device__ __forceinline__ bool must_rerun(Smem<DK>& sm) {
+    return __hip_atomic_load(&sm.sync.rerun, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0;
+}
+
 // PRE: the fused prologue (raw q, k projections and gate / beta logits).
 // NARROW: 16 rows of S per workgroup, for launches that leave CUs idle (the
 // rule is at the launch).  One wave scans (wave 0); wave 1 takes wave 2's
@@ -1523,11 +1528,12 @@ __global__ __launch_bounds__(512) void gdr_chunk_kernel(ChunkParams p) {
                                        p.heads, p.d_k, p.d_v, p.gate_is_alpha},
                                       u.seq, u.h, u.i0};
     }
-    __syncthreads();  // the only workgroup barrier: the chunk loops sync through sm.sync
+    __syncthreads();  // the only workgroup barrier ahead of the loops' end: they sync through sm.sync
 
     // Every role runs chunks 0 .. nch-1, unrolled by two so that buffer c & 1
     // is a compile-time constant.
-    if (w < (NARROW ? 1 : 2)) {
+    constexpr int kScans = NARROW ? 1 : 2;
+    if (w < kScans) {
         const int n = l & 15, g = l >> 4;
         const int i = u.i0 + 16 * w + n;
         const size_t srow = ((size_t(u.seq) * H + u.h) * dv + i) * dk;
@@ -1550,7 +1556,10 @@ __global__ __launch_bounds__(512) void gdr_chunk_kernel(ChunkParams p) {
             scan_chunk<DK, 0, NARROW>(p, sm, u, c, w, l, st);
             if (c + 1 < u.nch) scan_chunk<DK, 1, NARROW>(p, sm, u, c + 1, w, l, st);
         }
-        if (p.fin && i < dv) {
+        // a tile that will be recomputed leaves the final state alone: it may be
+        // the initial state's own buffer, from which the rerun starts
+        if constexpr (!PRE) __syncthreads();  // every role has left its loop and set its flag
+        if ((PRE || !must_rerun(sm)) && p.fin && i < dv) {
             const float f = exp2i(st.F);
 #pragma unroll
             for (int J = 0; J < NK; ++J) {
@@ -1609,9 +1618,9 @@ __global__ __launch_bounds__(512) void gdr_chunk_kernel(ChunkParams p) {
     }
 
     if constexpr (!PRE) {
-        __syncthreads();  // every role has left its loop and set its flag
-        const int rerun = __hip_atomic_load(&sm.sync.rerun, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (rerun != 0) {  // uniform over the workgroup
+        if (w >= kScans) __syncthreads();  // the scan waves' barrier ahead of their final state
+        // uniform over the workgroup; unlikely, or its code moves the loops' (1 % of their time)
+        if (__builtin_expect(must_rerun(sm), 0)) {
             // counted per 32 rows in both forms (the tiles of a head see the same
             // keys and gates, so they rerun together)
             if (threadIdx.x == 0 && u.i0 % kTV == 0) atomicAdd(&g_exact_reruns, 1u);

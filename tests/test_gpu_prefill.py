@@ -341,6 +341,24 @@ def test_out_of_domain_inputs_rerun_exactly(device, case):
     _check(w, o, fin, BF16_TOL, tag=f"{case}, chunked with exact rerun")
 
 
+@pytest.mark.parametrize("n_seqs", [2, 40])
+@pytest.mark.parametrize("case", OUT_OF_DOMAIN)
+def test_out_of_domain_state_in_place(device, case, n_seqs):
+    """final_state may be the initial_state buffer also where a tile is
+    recomputed: the rerun starts from the initial state, so outputs and final
+    states equal those of separate buffers bit for bit, with workgroups of 16
+    state rows (2 sequences: 24 of them) and of 32 (40 sequences: 240)."""
+    w = Prefill(heads=2, d_k=128, d_v=96, lengths=[70, 130] + [20] * (n_seqs - 2), dtype=torch.bfloat16,
+                device=device, state_std=0.5)
+    _leave_domain(w, case, seq=1, head=1)
+    o_sep, fin_sep = w.run(algo="chunked", reruns=3)
+    _check(w, o_sep, fin_sep, BF16_TOL, tag=f"{case}, separate buffers")
+    w.init = w.init.clone()
+    o_in, fin_in = w.run(algo="chunked", reruns=3, final_state=w.init)
+    assert fin_in.data_ptr() == w.init.data_ptr()
+    assert torch.equal(o_in, o_sep) and torch.equal(fin_in, fin_sep)
+
+
 def test_out_of_domain_dense_every_unit(device):
     """A dense batch in which every unit leaves the domain (q element 7e4 in
     every (batch, head)): every workgroup reruns, and all match the oracle;
