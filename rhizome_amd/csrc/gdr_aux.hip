@@ -604,9 +604,12 @@ hipError_t pick_rows(const P& p, int rows, int n, bool vec, hipStream_t st) {
 // sequences of one token, 6144 bf16 channels, 62 us in spans of 16 tokens
 // (every carried state another round trip of scalar accesses), 32 us with the
 // states read 16 bytes at a time, below the call's 17.6 us on the host in
-// spans of one token; conv1d 60.5 against 10.6 us.
-static int conv_span_len(const int32_t* cu, int seq_len, int most) {
-    return !cu && seq_len > 0 && seq_len < most ? seq_len : most;
+// spans of one token; conv1d 60.5 against 10.6 us.  Not where the shorter spans
+// are more blocks than a grid of 256 threads each can hold.
+static int conv_span_len(const int32_t* cu, int seq_len, int total, int ncb, int most) {
+    if (cu || seq_len <= 0 || seq_len >= most) return most;
+    const int64_t blocks = (int64_t)ncb * ((total + seq_len - 1) / seq_len);
+    return blocks * 256 <= UINT32_MAX ? seq_len : most;
 }
 
 // Whether a batch can hold empty sequences (their final state is written by
@@ -622,7 +625,7 @@ hipError_t launch_conv1d(const rhz_conv1d_args& a, hipStream_t st) {
     const int per_thread = vec ? nvec : 1;
     const int ncb = (a.channels / per_thread + 255) / 256;
     if (total > 0) {
-        const int span = conv_span_len(a.cu_seqlens, a.seq_len, kConvSpan);
+        const int span = conv_span_len(a.cu_seqlens, a.seq_len, total, ncb, kConvSpan);
         const dim3 grid((unsigned)((long)ncb * ((total + span - 1) / span)));
         if (a.dtype == RHZ_F32) {
             if (vec) hipLaunchKernelGGL((conv1d_kernel<float, true>), grid, dim3(256), 0, st, p, total, ncb, span);
@@ -661,7 +664,7 @@ hipError_t launch_conv_prepare(const rhz_gdr_conv_prepare_args& a, hipStream_t s
     const int g = a.d_k / n;
     const int ncb = (C / n + 255) / 256;
     if (total > 0) {
-        const int span = conv_span_len(a.cu_seqlens, a.seq_len, kConvPrepSpan);
+        const int span = conv_span_len(a.cu_seqlens, a.seq_len, total, ncb, kConvPrepSpan);
         const dim3 grid((unsigned)((long)ncb * ((total + span - 1) / span)));
 #define RHZ_CONV_PREP(T, G) hipLaunchKernelGGL((conv_prepare_kernel<T, G>), grid, dim3(256), 0, st, p, total, ncb, span)
         if (a.dtype == RHZ_F32) {

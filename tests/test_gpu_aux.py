@@ -517,3 +517,38 @@ def test_conv_short_sequences(device, dtype, tol, B, T, state):
     for got, ref in ((q, unit(yq) * d ** 0.5), (k, unit(yk)), (v, yv), (beta, torch.sigmoid(lg.double()))):
         check_close(host(got), ref.cpu().numpy(), tol, "conv_prepare")
     assert torch.equal(fin, fin_ref)
+
+
+@pytest.mark.parametrize("state", [False, True])
+def test_conv_more_sequences_than_blocks(device, state):
+    """Dense batches of more one-token sequences than a grid of 256-thread
+    blocks holds (2^32 / 256): conv1d and conv_prepare take them in longer
+    spans."""
+    B = (1 << 24) + 3
+    gen = torch.Generator(device=device).manual_seed(5)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=device)  # noqa: E731
+
+    def ref(x, w, bias, init):
+        xx = [x] if init is None else [*init.unbind(-1), x]
+        return bias + sum(w[:, 4 - len(xx) + j] * t for j, t in enumerate(xx))
+
+    x, w, bias = rand(B, 1, 1), rand(1, 4), rand(1)
+    init = rand(B, 1, 3) if state else None
+    y, fin = rhizome_amd.causal_conv1d(x, w, bias, initial_state=init, output_final_state=True)
+    # four products and four sums of N(0, 1) values in fp32
+    assert float((y[:, 0] - ref(x[:, 0], w, bias, init)).abs().max()) < 1e-4
+    past = torch.zeros(B, 1, 2, device=device) if init is None else init[..., 1:]
+    assert torch.equal(fin, torch.cat([past, x], -1))
+    del x, init, y, fin, past
+    d = 4
+    C = 3 * d
+    x, w, bias, lg, a = rand(B, 1, C), rand(C, 4), rand(C), rand(B, 1, 1), rand(1)
+    init = rand(B, C, 3) if state else None
+    q, k, v, beta, g, fin = rhizome_amd.conv_prepare(x, w, bias, lg, lg, a, heads=1, d_k=d, d_v=d, initial_state=init)
+    want = ref(x[:, 0], w, bias, init)
+    assert float((v[:, 0, 0] - want[:, 2 * d:]).abs().max()) < 1e-4
+    # unit rows: a relative error below 1e-5 in the convolution, unless it cancels (rows below 1e-2 left out)
+    for got, y in ((q / d ** 0.5, want[:, :d]), (k, want[:, d:2 * d])):
+        n = y.norm(dim=-1)
+        assert float(((got[:, 0, 0] - y / n[:, None]).abs().amax(-1) * (n > 1e-2)).max()) < 1e-2
+    assert float((beta - torch.sigmoid(lg)).abs().max()) < 1e-5
