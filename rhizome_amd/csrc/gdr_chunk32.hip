@@ -78,6 +78,7 @@ struct Chunk32Params {
     SeqParams sp;
     int units, n_tiles;
     int skip_short;  // the recurrence kernel runs the short sequences
+    int first;       // the launch's first workgroup
 };
 
 // Key columns of the operands.  Lane (m, g) = (lane & 15, lane >> 4).
@@ -746,7 +747,7 @@ __global__ __launch_bounds__(512, 2) void gdr_chunk32_kernel(Chunk32Params cp) {
     Smem32<DK>& sm = smu.chunk;
     const SeqParams& p = cp.sp;
     int unit, tile;
-    map_block(blockIdx.x, cp.units, cp.n_tiles, unit, tile);
+    map_block(cp.first + int(blockIdx.x), cp.units, cp.n_tiles, unit, tile);
     Unit32 u;
     u.seq = unit / p.heads;
     u.h = unit - u.seq * p.heads;
@@ -797,7 +798,7 @@ bool chunk32_supported(const rhz_gdr_prefill_args& a) {
 hipError_t launch_chunk32(const rhz_gdr_prefill_args& a, hipStream_t st) {
     Chunk32Params cp{{a.q, a.k, a.v, a.gate, a.beta, a.cu_seqlens, a.initial_state, a.final_state, a.o, a.seq_len,
                       a.heads, a.d_k, a.d_v, a.gate_kind == RHZ_GATE_ALPHA},
-                     a.batch * a.heads, (a.d_v + kRows - 1) / kRows, 0};
+                     a.batch * a.heads, (a.d_v + kRows - 1) / kRows, 0, 0};
     // A pack of mostly short sequences that more than fills the chip's 256 CUs:
     // the short ones run in the recurrence's own kernel, two of whose
     // workgroups share a CU where this kernel's LDS leaves room for one, and
@@ -809,14 +810,23 @@ hipError_t launch_chunk32(const rhz_gdr_prefill_args& a, hipStream_t st) {
         if (e != hipSuccess || a.seq_len <= kShortLen) return e;
         cp.skip_short = 1;
     }
-    const dim3 grid(cp.units * cp.n_tiles);
-    if (a.d_k <= 32)
-        hipLaunchKernelGGL(gdr_chunk32_kernel<32>, grid, dim3(512), 0, st, cp);
-    else if (a.d_k <= 64)
-        hipLaunchKernelGGL(gdr_chunk32_kernel<64>, grid, dim3(512), 0, st, cp);
-    else
-        hipLaunchKernelGGL(gdr_chunk32_kernel<128>, grid, dim3(512), 0, st, cp);
-    return hipGetLastError();
+    // A grid holds less than 2^32 work-items (the runtime truncates a larger one
+    // without an error): whole rounds over the XCDs of as many as fit.
+    constexpr int kMost = int(UINT32_MAX / 512) & ~7;
+    const int blocks = cp.units * cp.n_tiles;
+    hipError_t e = hipSuccess;
+    for (int64_t first = 0; first < blocks && e == hipSuccess; first += kMost) {
+        cp.first = int(first);
+        const dim3 grid(blocks - first > kMost ? kMost : int(blocks - first));
+        if (a.d_k <= 32)
+            hipLaunchKernelGGL(gdr_chunk32_kernel<32>, grid, dim3(512), 0, st, cp);
+        else if (a.d_k <= 64)
+            hipLaunchKernelGGL(gdr_chunk32_kernel<64>, grid, dim3(512), 0, st, cp);
+        else
+            hipLaunchKernelGGL(gdr_chunk32_kernel<128>, grid, dim3(512), 0, st, cp);
+        e = hipGetLastError();
+    }
+    return e;
 }
 
 }  // namespace rhz

@@ -177,3 +177,26 @@ def test_out_of_domain_is_the_recurrence(device, case, in_place):
         if not same:  # a tile without the value: the chunked result
             assert torch.equal(a, want_o[47:, 1, i0:i0 + 32]) and torch.equal(fa, want_f[1, 1, i0:i0 + 32])
     assert touched >= 1
+
+
+def test_more_workgroups_than_a_grid_holds(device):
+    """A pack of one-token sequences and a long one after them, in more
+    workgroups than a grid of 512 threads each holds (2^32 / 512): one token's
+    output and state in closed form, the long sequence as when run alone."""
+    import rhizome_amd
+
+    N, H, dk, dv, T = 1 << 18, 16, 4, 36, 81
+    gen = torch.Generator(device=device).manual_seed(7)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=device)  # noqa: E731
+    q, k, v = rand(N + T, H, dk), rand(N + T, H, dk), rand(N + T, H, dv)
+    k /= k.norm(dim=-1, keepdim=True)
+    g, beta = -torch.nn.functional.softplus(rand(N + T, H)), torch.sigmoid(rand(N + T, H))
+    cu = torch.cat([torch.arange(N + 1), torch.tensor([N + T])]).int().to(device)
+    o, fin = rhizome_amd.prefill(q, k, v, g, beta, cu_seqlens=cu)
+    bv = beta[:N, :, None] * v[:N]
+    # sums of four products of N(0, 1) values in fp32
+    assert float((o[:N] - bv * (k[:N] * q[:N]).sum(-1, keepdim=True)).abs().max()) < 1e-4
+    assert float((fin[:N] - bv[..., None] * k[:N, :, None]).abs().max()) < 1e-5
+    alone = torch.tensor([0, T], dtype=torch.int32, device=device)
+    o1, f1 = rhizome_amd.prefill(q[N:], k[N:], v[N:], g[N:], beta[N:], cu_seqlens=alone)
+    assert torch.equal(o[N:], o1) and torch.equal(fin[N], f1[0])
