@@ -13,6 +13,7 @@
 //   rmsnorm_kernel   RMSNorm of rows with a learned scale (norm.rs:8-13),
 //                    the per-head norm of the op's output (norm.rs:48-59).
 
+#include <algorithm>
 #include <type_traits>
 
 #include "gdr_device.hpp"
@@ -231,15 +232,20 @@ __device__ __forceinline__ void conv_span(const ConvParams& p, int total, int nc
     // before a sequence start the values come from its state, or are zero
     float a[3][N];
     auto window = [&](int seq, int start, int t) {  // before position t of the sequence from `start` on
-        float st[N][3];
-        if (t - 3 < start) {
-            if (p.init) {
-                load_conv_state<N>(p.init, ((long)seq * C + c) * 3, st);
-            } else {
+        if (!p.init) {  // uniform
 #pragma unroll
-                for (int e = 0; e < N; ++e) st[e][0] = st[e][1] = st[e][2] = 0.f;
+            for (int j = 0; j < 3; ++j) {
+                if (t - 3 + j >= start) {
+                    V::load(x + (t - 3 + j) * C + c, a[j]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < N; ++e) a[j][e] = 0.f;
+                }
             }
+            return;
         }
+        float st[N][3];
+        if (t - 3 < start) load_conv_state<N>(p.init, ((long)seq * C + c) * 3, st);
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             const int pos = t - 3 + j;
@@ -252,12 +258,12 @@ __device__ __forceinline__ void conv_span(const ConvParams& p, int total, int nc
             }
         }
     };
-    window(s, s0, t0);
     // every input of the span first, so that its loads overlap
     typename V::Raw xs[SPAN];
 #pragma unroll
     for (int i = 0; i < SPAN; ++i)
         if (t0 + i < t1) xs[i] = V::load_raw(x + (t0 + i) * C + c);
+    window(s, s0, t0);
 #pragma unroll
     for (int i = 0; i < SPAN; ++i) {
         const int t = t0 + i;
@@ -598,18 +604,38 @@ hipError_t pick_rows(const P& p, int rows, int n, bool vec, hipStream_t st) {
 
 }  // namespace
 
-// Tokens per span: dense sequences shorter than a span get spans of their own
-// length, so that a block meets one sequence and its one carried state
-// instead of up to `most` of them one after the other: conv_prepare on 64
-// sequences of one token, 6144 bf16 channels, 62 us in spans of 16 tokens
-// (every carried state another round trip of scalar accesses), 32 us with the
-// states read 16 bytes at a time, below the call's 17.6 us on the host in
-// spans of one token; conv1d 60.5 against 10.6 us.  Not where the shorter spans
-// are more blocks than a grid of 256 threads each can hold.
-static int conv_span_len(const int32_t* cu, int seq_len, int total, int ncb, int most) {
-    if (cu || seq_len <= 0 || seq_len >= most) return most;
-    const int64_t blocks = (int64_t)ncb * ((total + seq_len - 1) / seq_len);
-    return blocks * 256 <= UINT32_MAX ? seq_len : most;
+// Tokens per span of a dense batch (`most` for packs and for sequences of
+// `most` tokens or more).  Shorter sequences get spans of their own length,
+// so that a block meets one sequence instead of up to `most` one after the
+// other, where that does not cost more than it gives:
+// - With carried states every further sequence of a span is another round
+//   trip (4096 sequences of one token, 6144 bf16 channels, conv1d: 208 us in
+//   spans of one token, 292 in spans of 16; 64 sequences, conv_prepare: 9.4
+//   and 62).  Only blocks of less than half a wave of channels are bound by
+//   their number beyond 8192 (32768 sequences, 64 channels: 62 and 50 us).
+// - Without states a span's next sequence costs nothing, and each block reads
+//   20 bytes of weights and bias per channel: spans of less than 32 bytes per
+//   channel are for grids that leave the chip idle (conv1d, one token, 6144
+//   bf16 channels: 512 sequences 15 us in spans of one token, 20 in spans of
+//   16; 4096 sequences 89 and 31).  1024 blocks are four per CU; blocks of
+//   less than a wave of channels pay up to 4096 (4096 sequences of 8 channels:
+//   10 and 20 us; 32768: 49 and 24).
+// - A grid of 256-thread blocks holds less than 2^24 of them (the runtime
+//   truncates a larger one without an error).
+constexpr int64_t kMaxBlocks = UINT32_MAX / 256;
+static int conv_span_len(const ConvParams& p, int elem, int total, int ncb, int per_thread, int most) {
+    const int len = p.seq_len, active = p.C / per_thread;
+    if (p.cu || len <= 0 || len >= most) return most;
+    const auto blocks = [&](int span) { return (int64_t)ncb * ((total + span - 1) / span); };
+    int64_t target = kMaxBlocks;
+    if (p.init) {
+        if (active < 32) target = 8192;
+    } else if (len * elem < 32) {
+        target = active < 64 ? 4096 : 1024;
+    }
+    const int m = int(std::min<int64_t>((blocks(len) + target - 1) / target, most));  // sequences per span
+    const int span = p.init ? len * std::min(m, most / len) : std::min(len * m, most);
+    return blocks(span) <= kMaxBlocks ? span : most;
 }
 
 // Whether a batch can hold empty sequences (their final state is written by
@@ -625,7 +651,7 @@ hipError_t launch_conv1d(const rhz_conv1d_args& a, hipStream_t st) {
     const int per_thread = vec ? nvec : 1;
     const int ncb = (a.channels / per_thread + 255) / 256;
     if (total > 0) {
-        const int span = conv_span_len(a.cu_seqlens, a.seq_len, total, ncb, kConvSpan);
+        const int span = conv_span_len(p, a.dtype == RHZ_F32 ? 4 : 2, total, ncb, per_thread, kConvSpan);
         const dim3 grid((unsigned)((long)ncb * ((total + span - 1) / span)));
         if (a.dtype == RHZ_F32) {
             if (vec) hipLaunchKernelGGL((conv1d_kernel<float, true>), grid, dim3(256), 0, st, p, total, ncb, span);
@@ -664,7 +690,7 @@ hipError_t launch_conv_prepare(const rhz_gdr_conv_prepare_args& a, hipStream_t s
     const int g = a.d_k / n;
     const int ncb = (C / n + 255) / 256;
     if (total > 0) {
-        const int span = conv_span_len(a.cu_seqlens, a.seq_len, total, ncb, kConvPrepSpan);
+        const int span = conv_span_len(p.conv, a.dtype == RHZ_F32 ? 4 : 2, total, ncb, n, kConvPrepSpan);
         const dim3 grid((unsigned)((long)ncb * ((total + span - 1) / span)));
 #define RHZ_CONV_PREP(T, G) hipLaunchKernelGGL((conv_prepare_kernel<T, G>), grid, dim3(256), 0, st, p, total, ncb, span)
         if (a.dtype == RHZ_F32) {

@@ -552,3 +552,33 @@ def test_conv_more_sequences_than_blocks(device, state):
         n = y.norm(dim=-1)
         assert float(((got[:, 0, 0] - y / n[:, None]).abs().amax(-1) * (n > 1e-2)).max()) < 1e-2
     assert float((beta - torch.sigmoid(lg)).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("dtype,tol", PATHS)
+@pytest.mark.parametrize("B,T,H,d", [(4099, 1, 1, 64), (1500, 1, 3, 64), (700, 3, 3, 64), (2200, 2, 1, 64), (600, 7, 3, 64),
+                                     (700, 9, 3, 64), (600, 15, 3, 64), (9001, 1, 1, 16)])
+@pytest.mark.parametrize("state", [False, True])
+def test_conv_spans_of_several_short_sequences(device, dtype, tol, B, T, H, d, state):
+    """Dense batches whose spans hold several sequences, whole or split: more
+    one-sequence spans than 1024 blocks (4096 and 8192 of less than a wave and
+    half a wave of channels), with and without carried states, against f64."""
+    C = 3 * H * d
+    gen = torch.Generator(device=device).manual_seed(B + T)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=device)  # noqa: E731
+    x, w, bias, a, lg = rand(B, T, C).to(dtype), rand(C, 4), rand(C), rand(H), rand(B, T, H)
+    init = rand(B, C, 3) if state else None
+    past = torch.zeros(B, 3, C, device=device) if init is None else init.transpose(1, 2)
+    xx = torch.cat([past.double(), x.double()], 1)
+    y = bias.double() + sum(w[:, j].double() * xx[:, j:j + T] for j in range(4))
+    fin_ref = xx[:, T:].transpose(1, 2).float()
+    host = lambda t: t.float().cpu().numpy()  # noqa: E731
+    out, fin = rhizome_amd.causal_conv1d(x, w, bias, initial_state=init, output_final_state=True)
+    check_close(host(out), y.cpu().numpy(), tol, "conv1d")
+    assert torch.equal(fin, fin_ref)
+    q, k, v, beta, g, fin = rhizome_amd.conv_prepare(x, w, bias, lg, lg, a, heads=H, d_k=d, d_v=d, initial_state=init,
+                                                     output_final_state=True)
+    yq, yk, yv = (y[..., i * H * d:(i + 1) * H * d].reshape(B, T, H, d) for i in range(3))
+    unit = lambda t: t / t.norm(dim=-1, keepdim=True)  # noqa: E731
+    for got, ref in ((q, unit(yq) * d ** 0.5), (k, unit(yk)), (v, yv), (beta, torch.sigmoid(lg.double()))):
+        check_close(host(got), ref.cpu().numpy(), tol, "conv_prepare")
+    assert torch.equal(fin, fin_ref)
