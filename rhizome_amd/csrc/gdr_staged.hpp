@@ -124,19 +124,21 @@ __device__ __forceinline__ float dot_lane(const float (&a)[VPL], const float (&b
 }
 
 // The staging layout of NW computing waves whose rows of S each go to LPR
-// lanes holding VPL columns: DKP key columns, RPB rows per workgroup.
-template <int LPR, int VPL = 16, int NW = kStageWaves>
+// lanes holding VPL columns: DKP key columns, RPB rows per workgroup.  The
+// first NS waves of the workgroup stage (more than compute where a wave's rows
+// are many: the results are the same).
+template <int LPR, int VPL = 16, int NW = kStageWaves, int NS = NW>
 struct StageShape {
     static constexpr int DKP = VPL * LPR;        // padded key width
     static constexpr int RPW = 64 / LPR;         // rows per wave
     static constexpr int RPB = NW * RPW;         // state rows per workgroup
-    static constexpr int THREADS = NW * kWave;
+    static constexpr int THREADS = NS * kWave;   // threads that stage
     static constexpr int PPT = DKP / 4;          // float4 pieces of one position's k (or q)
     static constexpr int KQ4 = kStageTokens * PPT;       // float4 pieces of a block's k (or q)
     static constexpr int V4 = kStageTokens * RPB / 4;    // float4 pieces of a block's v
     static constexpr int NKQ = (KQ4 + THREADS - 1) / THREADS;
     static constexpr int NV = (V4 + THREADS - 1) / THREADS;
-    static_assert(VPL % 4 == 0 && VPL * LPR >= 4 && PPT <= 32, "supported staging shapes");
+    static_assert(VPL % 4 == 0 && VPL * LPR >= 4 && PPT <= 32 && NS >= NW, "supported staging shapes");
 };
 
 template <int LPR, int VPL = 16, int NW = kStageWaves>
@@ -154,17 +156,17 @@ struct StageSmem {
 // write.  Piece m of thread j is float4 number f = j + THREADS m of the
 // block's row-major [token][DKP] k (and q) tile; v likewise over
 // [token][RPB].
-template <int LPR, int VPL = 16, int NW = kStageWaves>
+template <int LPR, int VPL = 16, int NW = kStageWaves, int NS = NW>
 struct StageRegs {
-    using Shape = StageShape<LPR, VPL, NW>;
+    using Shape = StageShape<LPR, VPL, NW, NS>;
     float4 k[Shape::NKQ], q[Shape::NKQ], v[Shape::NV];
     float g, b;
 };
 
-template <int LPR, int VPL, int NW, typename T>
+template <int LPR, int VPL, int NW, int NS, typename T>
 __device__ __forceinline__ void stage_load(const SeqParams& p, int h, int i0, int tb, int len, int j,
-                                           StageRegs<LPR, VPL, NW>& r) {
-    using S = StageShape<LPR, VPL, NW>;
+                                           StageRegs<LPR, VPL, NW, NS>& r) {
+    using S = StageShape<LPR, VPL, NW, NS>;
     const long H = p.heads;
     const T* kp = static_cast<const T*>(p.k);
     const T* qp = static_cast<const T*>(p.q);
@@ -193,10 +195,10 @@ __device__ __forceinline__ void stage_load(const SeqParams& p, int h, int i0, in
 
 // Writes a block from registers to LDS buffer B, with alpha, beta and k.q of
 // every position.  Positions past the sequence's end hold zeros.
-template <int LPR, int VPL, int NW>
+template <int LPR, int VPL, int NW, int NS>
 __device__ __forceinline__ void stage_store(const SeqParams& p, StageSmem<LPR, VPL, NW>& sm, int B, int j,
-                                            const StageRegs<LPR, VPL, NW>& r) {
-    using S = StageShape<LPR, VPL, NW>;
+                                            const StageRegs<LPR, VPL, NW, NS>& r) {
+    using S = StageShape<LPR, VPL, NW, NS>;
     constexpr int PPT = S::PPT;  // a position's pieces: a group of PPT consecutive threads
 #pragma unroll
     for (int m = 0; m < S::NKQ; ++m) {
@@ -226,22 +228,22 @@ __device__ __forceinline__ void stage_store(const SeqParams& p, StageSmem<LPR, V
 
 // Rows i0 .. i0 + RPB - 1 (those below d_v) of sequence `seq`, head h,
 // carried through the whole sequence from the initial state (zero without
-// one): o written for every position, the final state at the end.  Threads
-// j < THREADS compute; a workgroup's further threads only take part in its
-// barriers, so every thread of the workgroup must call this.  Every thread
-// loads its share of block b + 1 -- k and q rows of the head, the rows' v,
-// the gates -- into registers while the waves run block b from LDS, then
-// writes it to the other LDS buffer together with k.q of each position
+// one): o written for every position, the final state at the end.  The first
+// NW waves compute, the first NS stage; a workgroup's further threads only
+// take part in its barriers, so every thread of the workgroup must call this.
+// Every staging thread loads its share of block b + 1 -- k and q rows of the
+// head, the rows' v, the gates -- into registers while the waves run block b
+// from LDS, then writes it to the other LDS buffer together with k.q of each position
 // (summed once per workgroup instead of once per row).  A wave then reads
 // each position's k and q from LDS, sums S_i.k and S_i.q over its row's
 // lanes by DPP, and updates its rows.  Lane li of a row's group holds
 // columns c*4*LPR + 4*li + e (c < VPL/4, e < 4).
-template <int LPR, typename T, int VPL = 16, int NW = kStageWaves>
+template <int LPR, typename T, int VPL = 16, int NW = kStageWaves, int NS = NW>
 __device__ __forceinline__ void staged_rows(const SeqParams& p, StageSmem<LPR, VPL, NW>& sm, int seq, int h,
                                             int i0, int j) {
-    using Sh = StageShape<LPR, VPL, NW>;
+    using Sh = StageShape<LPR, VPL, NW, NS>;
     constexpr int RPW = Sh::RPW;
-    const bool active = j < Sh::THREADS;  // uniform per wave
+    const bool active = j < NW * kWave, stages = j < Sh::THREADS;  // uniform per wave
     const int lane = j & 63, w = j >> 6;
     const int li = lane % LPR;
     const int rr = w * RPW + lane / LPR;  // row within the block of rows
@@ -263,10 +265,10 @@ __device__ __forceinline__ void staged_rows(const SeqParams& p, StageSmem<LPR, V
     }
     T* op = static_cast<T*>(p.o);
 
-    StageRegs<LPR, VPL, NW> regs;
-    if (nb > 0 && active) {
-        stage_load<LPR, VPL, NW, T>(p, h, i0, t0, min(kStageTokens, t1 - t0), j, regs);
-        stage_store<LPR, VPL, NW>(p, sm, 0, j, regs);
+    StageRegs<LPR, VPL, NW, NS> regs;
+    if (nb > 0 && stages) {
+        stage_load<LPR, VPL, NW, NS, T>(p, h, i0, t0, min(kStageTokens, t1 - t0), j, regs);
+        stage_store<LPR, VPL, NW, NS>(p, sm, 0, j, regs);
     }
     __syncthreads();
     T* orow = op + (long)h * dv + r;  // o of position t at orow + t * H * dv
@@ -276,10 +278,10 @@ __device__ __forceinline__ void staged_rows(const SeqParams& p, StageSmem<LPR, V
         const int tb = t0 + b * kStageTokens;
         const int len = min(kStageTokens, t1 - tb);
         const bool more = b + 1 < nb;  // uniform
+        if (more && stages)
+            stage_load<LPR, VPL, NW, NS, T>(p, h, i0, tb + kStageTokens, min(kStageTokens, t1 - tb - kStageTokens), j,
+                                            regs);
         if (active) {
-            if (more)
-                stage_load<LPR, VPL, NW, T>(p, h, i0, tb + kStageTokens, min(kStageTokens, t1 - tb - kStageTokens),
-                                            j, regs);
             for (int tt = 0; tt < len; ++tt) {
                 float kr[VPL], qr[VPL];
 #pragma unroll
@@ -303,10 +305,10 @@ __device__ __forceinline__ void staged_rows(const SeqParams& p, StageSmem<LPR, V
                 for (int e = 0; e < VPL; ++e) s[e] = fmaf(gb.x, s[e], c * kr[e]);
                 if (li == 0 && row_ok) Elem<T>::store(orow, (long)(tb + tt) * ostride, oi);
             }
-            // buffer B ^ 1 was last read in block b - 1, which every wave has
-            // left (the barrier below closed it)
-            if (more) stage_store<LPR, VPL, NW>(p, sm, B ^ 1, j, regs);
         }
+        // buffer B ^ 1 was last read in block b - 1, which every wave has
+        // left (the barrier below closed it)
+        if (more && stages) stage_store<LPR, VPL, NW, NS>(p, sm, B ^ 1, j, regs);
         __syncthreads();
     }
     if (p.fin && row_ok) {
