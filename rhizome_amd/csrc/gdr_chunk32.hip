@@ -137,12 +137,30 @@ struct Smem32 {
     int rerun;  // an input left the domain
 };
 
+// The recurrence in this kernel (short sequences and reruns), in the lanes per
+// row and columns per lane that the recurrence's own kernel has for these d_k:
+// equal to it bit for bit.  The tile's rows take one, two or eight of the
+// workgroup's waves; all of them stage.
+template <int DK>
+struct Recurrence32 {
+    static constexpr int LPR = DK == 128 ? 16 : DK / 16;
+    static constexpr int VPL = DK / LPR;
+    static constexpr int NW = kRows * LPR / kWave;
+    using Smem = StageSmem<LPR, VPL, NW>;
+    static_assert(Smem::RPB == kRows && Smem::DKP == DK, "the recurrence covers the tile");
+};
+
 template <int DK>
 union KernelSmem32 {
     Smem32<DK> chunk;
-    StageSmem<16, 8, 8> rerun;  // 128 key columns, 32 rows
+    typename Recurrence32<DK>::Smem rec;
 };
-static_assert(StageSmem<16, 8, 8>::RPB == kRows && StageShape<16, 8, 8>::THREADS == 512, "the rerun covers the tile");
+
+template <int DK>
+__device__ __forceinline__ void recurrence32(const SeqParams& p, KernelSmem32<DK>& smu, int seq, int h, int i0) {
+    using R = Recurrence32<DK>;
+    staged_rows<R::LPR, float, R::VPL, R::NW, 8>(p, smu.rec, seq, h, i0, threadIdx.x);
+}
 
 __device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 __device__ __forceinline__ void st4(float* p, f32x4 x) { *reinterpret_cast<f32x4*>(p) = x; }
@@ -755,7 +773,7 @@ __global__ __launch_bounds__(512, 2) void gdr_chunk32_kernel(Chunk32Params cp) {
     seq_bounds(p.cu_seqlens, u.seq, p.seq_len, u.tb, u.te);
     u.nch = (u.te - u.tb + kC - 1) / kC;
     if (u.te - u.tb <= kShortLen) {  // uniform
-        if (!cp.skip_short) staged_rows<16, float, 8, 8>(p, smu.rerun, u.seq, u.h, u.i0, threadIdx.x);
+        if (!cp.skip_short) recurrence32<DK>(p, smu, u.seq, u.h, u.i0);
         return;
     }
     const int l = threadIdx.x & 63;
@@ -780,7 +798,7 @@ __global__ __launch_bounds__(512, 2) void gdr_chunk32_kernel(Chunk32Params cp) {
     const int rerun = sm.rerun;
     if (rerun != 0) {  // uniform: set before the last barrier
         __syncthreads();  // every wave has read the flag: the LDS is free
-        staged_rows<16, float, 8, 8>(p, smu.rerun, u.seq, u.h, u.i0, threadIdx.x);
+        recurrence32<DK>(p, smu, u.seq, u.h, u.i0);
     }
 }
 
@@ -806,7 +824,7 @@ hipError_t launch_chunk32(const rhz_gdr_prefill_args& a, hipStream_t st) {
     // of 16 tokens each take 39 us, with it 22.  A sequence's arithmetic follows
     // from its own length in either case.
     if (a.cu_seqlens && a.seq_len / a.batch <= kShortLen && (int64_t)cp.units * cp.n_tiles > 256) {
-        const hipError_t e = launch_staged_short(cp.sp, a.batch * a.heads, kShortLen, st);
+        const hipError_t e = launch_staged_short(cp.sp, cp.units, kShortLen, st);
         if (e != hipSuccess || a.seq_len <= kShortLen) return e;
         cp.skip_short = 1;
     }

@@ -376,7 +376,8 @@ hipError_t recurrent_pick_lpr(const SeqParams& sp, int units, int dk, int dv, hi
 }
 
 template <typename T>
-hipError_t staged_pick_lpr(const SeqParams& sp, int units, int dk, int dv, hipStream_t st) {
+hipError_t staged_pick_lpr(const SeqParams& sp, int units, int dk, int dv, hipStream_t st,
+                           int max_len = INT32_MAX) {
     const int lpr = lanes_per_row(dk);
     if (lpr == 8) {
         // d_k in (64, 128]: 16 lanes of 8 columns per row and eight waves of
@@ -384,14 +385,14 @@ hipError_t staged_pick_lpr(const SeqParams& sp, int units, int dk, int dv, hipSt
         // other's latency along the position chain.
         using Sh = StageShape<16, 8, 8>;
         dim3 grid(units, (dv + Sh::RPB - 1) / Sh::RPB);
-        hipLaunchKernelGGL((gdr_staged_recurrent_kernel<16, T, 8, 8>), grid, dim3(Sh::THREADS), 0, st, sp, INT32_MAX);
+        hipLaunchKernelGGL((gdr_staged_recurrent_kernel<16, T, 8, 8>), grid, dim3(Sh::THREADS), 0, st, sp, max_len);
         return hipGetLastError();
     }
     const int rpb = kStageWaves * (64 / lpr);
     dim3 grid(units, (dv + rpb - 1) / rpb);
     switch (lpr) {
-        case 2: hipLaunchKernelGGL((gdr_staged_recurrent_kernel<2, T, 16, kStageWaves>), grid, dim3(kStageThreads), 0, st, sp, INT32_MAX); break;
-        default: hipLaunchKernelGGL((gdr_staged_recurrent_kernel<4, T, 16, kStageWaves>), grid, dim3(kStageThreads), 0, st, sp, INT32_MAX); break;
+        case 2: hipLaunchKernelGGL((gdr_staged_recurrent_kernel<2, T, 16, kStageWaves>), grid, dim3(kStageThreads), 0, st, sp, max_len); break;
+        default: hipLaunchKernelGGL((gdr_staged_recurrent_kernel<4, T, 16, kStageWaves>), grid, dim3(kStageThreads), 0, st, sp, max_len); break;
     }
     return hipGetLastError();
 }
@@ -399,10 +400,7 @@ hipError_t staged_pick_lpr(const SeqParams& sp, int units, int dk, int dv, hipSt
 }  // namespace
 
 hipError_t launch_staged_short(const SeqParams& sp, int units, int max_len, hipStream_t st) {
-    using Sh = StageShape<16, 8, 8>;
-    dim3 grid(units, (sp.d_v + Sh::RPB - 1) / Sh::RPB);
-    hipLaunchKernelGGL((gdr_staged_recurrent_kernel<16, float, 8, 8>), grid, dim3(Sh::THREADS), 0, st, sp, max_len);
-    return hipGetLastError();
+    return staged_pick_lpr<float>(sp, units, sp.d_k, sp.d_v, st, max_len);
 }
 
 hipError_t launch_decode(const rhz_gdr_decode_args& a, hipStream_t st) {

@@ -32,9 +32,8 @@ struct SeqParams {
     int seq_len, heads, d_k, d_v, gate_is_alpha;
 };
 
-// The recurrence over the sequences of up to max_len fp32 tokens, in the shape
-// that the 16-token chunked kernel's own runs of it have (d_k <= 128, tensors
-// and widths as that kernel takes them): equal bit for bit.
+// gdr_staged_recurrent_kernel over the sequences of up to max_len fp32 tokens
+// (d_k <= 128, tensors and widths as the 16-token chunked kernel takes them).
 hipError_t launch_staged_short(const SeqParams& sp, int units, int max_len, hipStream_t st);
 
 // The 16 columns of a row held by lane li of its group (zero outside [0, n)).

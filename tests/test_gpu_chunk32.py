@@ -35,7 +35,7 @@ SHAPES = [
     dict(batch=1, heads=9, seq_len=200, d_k=128, d_v=256),
     dict(lengths=[0, 1, 16, 0, 31, 64, 200, 5, 0], heads=2, d_k=128, d_v=96, state_std=0.5),
     dict(lengths=[33, 79, 128], heads=3, d_k=64, d_v=32, state_std=0.02),
-    # few tokens per sequence on average: the short ones in the recurrence's kernel
+    # mostly short sequences, in one launch
     dict(lengths=[64, 65, 0, 3, 100, 7, 1, 64, 130, 33], heads=2, d_k=128, d_v=40, state_std=0.3),
     dict(lengths=[5, 40], heads=2, d_k=32, d_v=64),
     dict(batch=1, heads=1, seq_len=3000, d_k=128, d_v=32, g_mean=-2.0, state_std=0.02),
@@ -86,6 +86,49 @@ def test_batch_invariant(device, d_k):
                                          initial_state=init)
             assert torch.equal(o1, o[a:b]) and torch.equal(f1[0], f[i])
             assert tail == 0 or torch.equal(f1[1:], init[1:])
+
+
+@pytest.mark.parametrize("d_k,d_v", [(20, 12), (32, 96), (64, 40), (100, 64), (128, 128)])
+@pytest.mark.parametrize("tail", [0, 300])
+def test_short_sequences_are_the_recurrence(device, d_k, d_v, tail):
+    """Sequences of up to 64 tokens: the same bits in a pack, in a pack large
+    enough for the recurrence's own launch (300 sequences more), in a dense
+    batch and under RECURRENT."""
+    import rhizome_amd
+
+    w = Prefill(lengths=[64, 17, 0, 1, 33, 64] + [1] * tail, heads=2, d_k=d_k, d_v=d_v, dtype=torch.float32,
+                device=device, state_std=0.3)
+    o, f = w.run()
+    ro, rf = w.run(algo="recurrent")
+    assert torch.equal(o, ro) and torch.equal(f, rf)
+    for i in (0, 1, 4):
+        a, b = int(w.cu[i]), int(w.cu[i + 1])
+        do, df = rhizome_amd.prefill(*(x[None, a:b].contiguous() for x in (w.q, w.k, w.v, w.g, w.beta)),
+                                     initial_state=w.init[i:i + 1].contiguous())
+        assert torch.equal(do[0], o[a:b]) and torch.equal(df[0], f[i])
+
+
+# short and long sequences in turn, more than 256 workgroups of 32 rows, and a
+# mean length of at most 64: the short ones go out in the recurrence's launch,
+# the others in the chunked one
+@pytest.mark.parametrize("d_k,d_v", [(32, 128), (64, 64), (128, 96)])
+def test_pack_in_two_launches(device, d_k, d_v):
+    import rhizome_amd
+
+    lengths = [0, 1, 63, 64, 65, 200, 5, 129, 0, 70, 16, 3, 40, 0, 2, 1] * 4
+    w = Prefill(lengths=lengths, heads=4, d_k=d_k, d_v=d_v, dtype=torch.float32, device=device, state_std=0.3)
+    assert len(lengths) * w.heads * ((d_v + 31) // 32) > 256 and w.n_tok // len(lengths) <= 64
+    o, f = w.run()
+    _check(w, o, f, f"two launches d_k={d_k}")
+    for i in range(len(lengths) - 16, len(lengths)):
+        a, b = int(w.cu[i]), int(w.cu[i + 1])
+        cu = torch.tensor([0, b - a], dtype=torch.int32, device=device)
+        if b > a:
+            o1, f1 = rhizome_amd.prefill(*(x[a:b] for x in (w.q, w.k, w.v, w.g, w.beta)), cu_seqlens=cu,
+                                         initial_state=w.init[i:i + 1].contiguous())
+            assert torch.equal(o1, o[a:b]) and torch.equal(f1[0], f[i])
+        else:
+            assert torch.equal(f[i], w.init[i])
 
 
 @pytest.mark.parametrize("m", [1, 16, 21, 64])
@@ -140,13 +183,14 @@ CASES = ["beta |k|^2 above 2", "beta -0.5", "alpha 1.05", "v inf", "v nan in the
 
 @pytest.mark.parametrize("in_place", [False, True])
 @pytest.mark.parametrize("case", CASES)
-def test_out_of_domain_is_the_recurrence(device, case, in_place):
+@pytest.mark.parametrize("d_k", [128, 64, 24])
+def test_out_of_domain_is_the_recurrence(device, case, in_place, d_k):
     """Inputs outside the op's domain or not finite, at the last token of a
     16-token chunk or at the first of a partial one, in one head: every other
     (sequence, head) is unchanged, and the head's tiles equal the recurrence
     bit for bit or the chunked result where they hold no such value (a value
     row's tile), also when the state is updated in place."""
-    kw = dict(heads=2, d_k=128, d_v=64, lengths=[47, 102], dtype=torch.float32, device=device, state_std=0.1)
+    kw = dict(heads=2, d_k=d_k, d_v=64, lengths=[47, 102], dtype=torch.float32, device=device, state_std=0.1)
     w, plain = Prefill(**kw), Prefill(**kw)
     if "3e38" in case:
         w.q *= 1e3
