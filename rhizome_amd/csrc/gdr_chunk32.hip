@@ -76,9 +76,9 @@ constexpr int kShortLen = 64;
 
 struct Chunk32Params {
     SeqParams sp;
-    int units, n_tiles;
-    int skip_short;  // the recurrence kernel runs the short sequences
-    int first;       // the launch's first workgroup
+    int batch, units, n_tiles;
+    int long_only;  // units count the sequences of more than kShortLen tokens (the recurrence kernel runs the others)
+    int first;      // the launch's first workgroup
 };
 
 // Key columns of the operands.  Lane (m, g) = (lane & 15, lane >> 4).
@@ -759,6 +759,35 @@ __device__ __forceinline__ void out32(const SeqParams& p, const Unit32& u, Smem3
     }
 }
 
+// The r-th sequence of a pack (from 0) among those of more than kShortLen
+// tokens, or -1.  Called by the whole workgroup; `scratch`, nine ints of LDS,
+// is free after the caller's next barrier.
+__device__ __forceinline__ int nth_long(const SeqParams& p, int batch, int r, int* scratch) {
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int base = 0; base < batch; base += 512) {
+        const int s = base + threadIdx.x;
+        bool is_long = false;
+        if (s < batch) {
+            int t0, t1;
+            seq_bounds(p.cu_seqlens, s, p.seq_len, t0, t1);
+            is_long = t1 - t0 > kShortLen;
+        }
+        const uint64_t m = __builtin_amdgcn_ballot_w64(is_long);
+        if (l == 0) scratch[w] = __popcll(m);
+        __syncthreads();
+        int before = __popcll(m & ((uint64_t(1) << l) - 1)), all = 0;
+        for (int i = 0; i < 8; ++i) {
+            before += i < w ? scratch[i] : 0;
+            all += scratch[i];
+        }
+        if (is_long && before == r) scratch[8] = s;
+        __syncthreads();
+        if (r < all) return scratch[8];  // uniform
+        r -= all;
+    }
+    return -1;
+}
+
 template <int DK>
 __global__ __launch_bounds__(512, 2) void gdr_chunk32_kernel(Chunk32Params cp) {
     __shared__ __align__(16) KernelSmem32<DK> smu;
@@ -770,10 +799,14 @@ __global__ __launch_bounds__(512, 2) void gdr_chunk32_kernel(Chunk32Params cp) {
     u.seq = unit / p.heads;
     u.h = unit - u.seq * p.heads;
     u.i0 = tile * kRows;
+    if (cp.long_only) {
+        u.seq = nth_long(p, cp.batch, u.seq, reinterpret_cast<int*>(&smu));
+        if (u.seq < 0) return;  // uniform
+    }
     seq_bounds(p.cu_seqlens, u.seq, p.seq_len, u.tb, u.te);
     u.nch = (u.te - u.tb + kC - 1) / kC;
     if (u.te - u.tb <= kShortLen) {  // uniform
-        if (!cp.skip_short) recurrence32<DK>(p, smu, u.seq, u.h, u.i0);
+        recurrence32<DK>(p, smu, u.seq, u.h, u.i0);
         return;
     }
     const int l = threadIdx.x & 63;
@@ -816,17 +849,21 @@ bool chunk32_supported(const rhz_gdr_prefill_args& a) {
 hipError_t launch_chunk32(const rhz_gdr_prefill_args& a, hipStream_t st) {
     Chunk32Params cp{{a.q, a.k, a.v, a.gate, a.beta, a.cu_seqlens, a.initial_state, a.final_state, a.o, a.seq_len,
                       a.heads, a.d_k, a.d_v, a.gate_kind == RHZ_GATE_ALPHA},
-                     a.batch * a.heads, (a.d_v + kRows - 1) / kRows, 0, 0};
+                     a.batch, a.batch * a.heads, (a.d_v + kRows - 1) / kRows, 0, 0};
     // A pack of mostly short sequences that more than fills the chip's 256 CUs:
-    // the short ones run in the recurrence's own kernel, two of whose
-    // workgroups share a CU where this kernel's LDS leaves room for one, and
-    // the rest here.  The second launch costs 4 us; without it 1024 workgroups
-    // of 16 tokens each take 39 us, with it 22.  A sequence's arithmetic follows
-    // from its own length in either case.
+    // the short ones run in the recurrence's own kernel, two or three of whose
+    // workgroups share a CU where this kernel's LDS leaves room for one, and the
+    // rest here, in as many workgroups as its tokens could need (each finds its
+    // sequence by counting; workgroups for every sequence, most of them with
+    // nothing to do, took 0.55 us per 256).  H=16 d=64, 1024 sequences of one
+    // token: 227 us in one launch, 154 with empty workgroups, 87 so.  A
+    // sequence's arithmetic follows from its own length in either case.
     if (a.cu_seqlens && a.seq_len / a.batch <= kShortLen && (int64_t)cp.units * cp.n_tiles > 256) {
         const hipError_t e = launch_staged_short(cp.sp, cp.units, kShortLen, st);
-        if (e != hipSuccess || a.seq_len <= kShortLen) return e;
-        cp.skip_short = 1;
+        const int most = a.seq_len / (kShortLen + 1);
+        if (e != hipSuccess || most == 0) return e;
+        cp.units = (most < a.batch ? most : a.batch) * a.heads;
+        cp.long_only = 1;
     }
     // A grid holds less than 2^32 work-items (the runtime truncates a larger one
     // without an error): whole rounds over the XCDs of as many as fit.
