@@ -52,7 +52,9 @@
 // beta |k|^2 outside [0, 2], or values that are not finite, where a product
 // with a masked zero would spread a NaN to earlier positions -- are noticed
 // as they pass, and the workgroup then recomputes its rows with the
-// token-sequential recurrence (staged_rows) in the same launch.
+// token-sequential recurrence (staged_rows) in the same launch: at once where a
+// key, gate or beta of the first 64 tokens is outside, else at the sequence's
+// end.
 
 #include "gdr_device.hpp"
 #include "gdr_internal.hpp"
@@ -174,6 +176,17 @@ __device__ __forceinline__ void period_end() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+}
+
+// The end of period 1.  True where wave 6 found an input of the first superblock
+// outside the domain in period 0: every wave then leaves the pipeline.  (No
+// flag is set in period 1, so all waves read the same.  A check at every
+// superblock cost sequences inside the domain 1 to 2 %.)
+template <int DK>
+__device__ __forceinline__ bool period1_leaves(Smem32<DK>& sm) {
+    const int rerun = sm.rerun;
+    period_end();
+    return __builtin_amdgcn_readfirstlane(rerun) != 0;
 }
 
 // The operand pieces of lane (m, g): row m of a K or Q tile.
@@ -331,7 +344,10 @@ __device__ __forceinline__ void loader32(const SeqParams& p, const Unit32& u, Sm
             if (c + 1 >= u.nch) break;
             stage32<DK>(p, u, sm, c + 1, j, r1);
             load32<DK>(p, u, c + 3, j, o, r1);
-            period_end();
+            if (c > 0)
+                period_end();
+            else if (period1_leaves(sm))
+                return;
         }
     }
     for (int i = 0; i < 4; ++i) period_end();
@@ -477,6 +493,7 @@ struct TWave {
     __device__ __forceinline__ void run() {
         constexpr int HB = NB / 2;
         const int nsb = (u.nch + 3) / 4;
+        bool leave = false;  // as period1_leaves
         if (nsb > 0) {  // superblock 0, in period 0
             load_gates(0);
             load_k(0, x0);
@@ -488,6 +505,8 @@ struct TWave {
             product(x0, 2, 4);
             product(x1, 3, 5);
             solve(0);
+            leave = __builtin_amdgcn_ballot_w64(bad) != 0;
+            flag32(sm, bad);
             load_gates(1);
         }
         period_end();
@@ -501,7 +520,7 @@ struct TWave {
                 acc.template mma<0, HB>(x0, x0);
             }
             period_end();
-            if (q + 1 >= last) break;
+            if (q + 1 >= last || (q == 1 && leave)) break;
             if (on) {
                 acc.template mma<HB, NB>(x0, x0);
                 load_k(4 * sb + 2, x0);
@@ -577,7 +596,7 @@ __device__ __forceinline__ void p_wave32(const Unit32& u, Smem32<DK>& sm, int l)
     In a, b;
     period_end();
     if (u.nch > 0) load(0, a);
-    period_end();
+    if (period1_leaves(sm)) return;
     for (int c = 0; c < u.nch; c += 2) {  // by two, so that the operands need no copies
         step(c, a, b);
         if (c + 1 < u.nch) step(c + 1, b, a);
@@ -618,7 +637,7 @@ __device__ __forceinline__ void scan32(const SeqParams& p, const Unit32& u, Smem
     f32x4 kx[NB];
     period_end();
     if (u.nch > 0) load_operand<DK>(sm.k[0], sig(n), g, kx);
-    period_end();
+    if (period1_leaves(sm)) return;
     for (int c = 0; c < u.nch; ++c) {
         const int slot = c & 3, sb = c & 7, B = c & 1;
 #pragma unroll
@@ -750,7 +769,9 @@ __device__ __forceinline__ void out32(const SeqParams& p, const Unit32& u, Smem3
         period_end();
     };
     In a, b;
-    for (int k = 0; k < 3; ++k) period_end();
+    period_end();
+    if (period1_leaves(sm)) return;
+    period_end();
     if (u.nch > 0) load(0, a);
     period_end();
     for (int c = 0; c < u.nch; c += 2) {
@@ -814,7 +835,7 @@ __global__ __launch_bounds__(512, 2) void gdr_chunk32_kernel(Chunk32Params cp) {
     if (threadIdx.x == 0) sm.rerun = 0;
     period_end();
 
-    // every role passes nch + 4 period ends
+    // every role passes nch + 4 period ends, or leaves after the second
     if (w < 2)
         scan32<DK>(p, u, sm, w, l);
     else if (w < 4)

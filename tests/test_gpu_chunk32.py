@@ -223,6 +223,27 @@ def test_out_of_domain_is_the_recurrence(device, case, in_place, d_k):
     assert touched >= 1
 
 
+@pytest.mark.parametrize("t", [0, 15, 63, 64, 127, 128, 250, 255, 256, 278, 280])
+@pytest.mark.parametrize("d_k", [128, 64, 32])
+def test_leaves_the_domain_anywhere(device, t, d_k):
+    """An input outside the domain in the first 64 tokens, where the pipeline
+    ends at once, and in every later superblock of 64: the recurrence's results
+    in its head, unchanged ones elsewhere, with the state updated in place too."""
+    T = 250 if t == 0 else 281  # 4 superblocks or 5, and a last chunk that is not full
+    kw = dict(heads=2, d_k=d_k, d_v=40, batch=1, seq_len=T, dtype=torch.float32, device=device, state_std=0.1)
+    w, plain = Prefill(**kw), Prefill(**kw)
+    t = min(t, T - 1)
+    w.beta[t, 0] = -0.25
+    want_o, want_f = plain.run()
+    ro, rf = w.run(algo="recurrent")
+    o, f = w.run()
+    w.init = w.init.clone()
+    oi, fi = w.run(final_state=w.init)
+    assert torch.equal(o, oi) and torch.equal(f, fi)
+    assert torch.equal(o[:, 0], ro[:, 0]) and torch.equal(f[:, 0], rf[:, 0])
+    assert torch.equal(o[:, 1], want_o[:, 1]) and torch.equal(f[:, 1], want_f[:, 1])
+
+
 def test_more_workgroups_than_a_grid_holds(device):
     """A pack of one-token sequences and a long one after them, in more
     workgroups than a grid of 512 threads each holds (2^32 / 512): one token's
