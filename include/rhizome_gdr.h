@@ -49,7 +49,8 @@ typedef enum rhz_status {
     RHZ_ERR_INVALID_ARG = 1, /* null pointer, bad dimension or size, bad enum */
     RHZ_ERR_UNSUPPORTED = 2, /* well-formed but not supported (dims, dtype, algo) */
     RHZ_ERR_WORKSPACE = 3,   /* workspace missing, too small or misaligned */
-    RHZ_ERR_HIP = 4          /* the HIP runtime reported an error */
+    RHZ_ERR_HIP = 4          /* the HIP runtime reported an error, or the call needs a grid
+                                of 2^32 work-items or more, which it cannot launch */
 } rhz_status;
 
 /* RHZ_F64 is accepted only as the output dtype of rhz_philox_fill. */

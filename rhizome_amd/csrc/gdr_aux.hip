@@ -652,7 +652,9 @@ hipError_t launch_conv1d(const rhz_conv1d_args& a, hipStream_t st) {
     const int ncb = (a.channels / per_thread + 255) / 256;
     if (total > 0) {
         const int span = conv_span_len(p, a.dtype == RHZ_F32 ? 4 : 2, total, ncb, per_thread, kConvSpan);
-        const dim3 grid((unsigned)((long)ncb * ((total + span - 1) / span)));
+        const int64_t blocks = (int64_t)ncb * ((total + span - 1) / span);
+        if (const hipError_t e = check_grid(blocks, 256); e != hipSuccess) return e;
+        const dim3 grid((unsigned)blocks);
         if (a.dtype == RHZ_F32) {
             if (vec) hipLaunchKernelGGL((conv1d_kernel<float, true>), grid, dim3(256), 0, st, p, total, ncb, span);
             else hipLaunchKernelGGL((conv1d_kernel<float, false>), grid, dim3(256), 0, st, p, total, ncb, span);
@@ -691,7 +693,9 @@ hipError_t launch_conv_prepare(const rhz_gdr_conv_prepare_args& a, hipStream_t s
     const int ncb = (C / n + 255) / 256;
     if (total > 0) {
         const int span = conv_span_len(p.conv, a.dtype == RHZ_F32 ? 4 : 2, total, ncb, n, kConvPrepSpan);
-        const dim3 grid((unsigned)((long)ncb * ((total + span - 1) / span)));
+        const int64_t blocks = (int64_t)ncb * ((total + span - 1) / span);
+        if (const hipError_t e = check_grid(blocks, 256); e != hipSuccess) return e;
+        const dim3 grid((unsigned)blocks);
 #define RHZ_CONV_PREP(T, G) hipLaunchKernelGGL((conv_prepare_kernel<T, G>), grid, dim3(256), 0, st, p, total, ncb, span)
         if (a.dtype == RHZ_F32) {
             switch (g) {

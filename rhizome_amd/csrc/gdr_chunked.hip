@@ -1808,6 +1808,7 @@ hipError_t launch_chunked_with(const rhz_gdr_prefill_args& a, hipStream_t st, in
     const int narrow_tiles = (a.d_v + kTVNarrow - 1) / kTVNarrow;
     const bool narrow = !pro && (int64_t)a.batch * a.heads * narrow_tiles <= kCUs;
     cp.n_tiles = narrow ? narrow_tiles : (a.d_v + kTV - 1) / kTV;
+    if (const hipError_t e = check_grid((int64_t)a.batch * a.heads * cp.n_tiles, 512); e != hipSuccess) return e;
     cp.spin_limit = spin_limit > 0 ? spin_limit : kSpinLimit;
     cp.order = nullptr;
     if (a.cu_seqlens) {

@@ -11,6 +11,12 @@
 
 namespace rhz {
 
+// Whether the runtime launches a grid of `blocks` workgroups of `threads` along
+// x as asked: it truncates one of 2^32 work-items or more without an error.
+inline hipError_t check_grid(int64_t blocks, int threads) {
+    return blocks * threads <= UINT32_MAX ? hipSuccess : hipErrorInvalidConfiguration;
+}
+
 // Token-sequential fp32 recurrence over a dense or packed batch.
 hipError_t launch_recurrent(const rhz_gdr_prefill_args& a, hipStream_t stream);
 

@@ -114,8 +114,10 @@ __global__ __launch_bounds__(256) void philox_unit_rows_kernel(uint64_t seed, ui
 hipError_t launch_philox_fill(int kind, uint64_t seed, uint64_t sid, int64_t count, int row_len, double mean,
                               double sd, int dtype, void* out, hipStream_t st) {
     if (count <= 0) return hipSuccess;
+    const int64_t items = kind == RHZ_FILL_UNIT_ROWS ? count / row_len : count;
+    if (const hipError_t e = check_grid((items + 255) / 256, 256); e != hipSuccess) return e;
     if (kind == RHZ_FILL_UNIT_ROWS) {
-        const int64_t rows = count / row_len;
+        const int64_t rows = items;
         hipLaunchKernelGGL(philox_unit_rows_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, st, seed,
                            sid, rows, row_len, dtype, out);
     } else {

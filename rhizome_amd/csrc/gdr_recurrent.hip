@@ -292,6 +292,7 @@ bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) %
 template <int LPR, int P, bool VEC, typename T, bool NTL = false>
 hipError_t decode_go(const StepParams& sp, int units, int dv, hipStream_t st) {
     constexpr int RPP = 256 / LPR;
+    if (const hipError_t e = check_grid(units, 256); e != hipSuccess) return e;
     dim3 grid(units, (dv + P * RPP - 1) / (P * RPP));
     hipLaunchKernelGGL((gdr_decode_kernel<LPR, P, VEC, T, NTL>), grid, dim3(256), 0, st, sp);
     return hipGetLastError();
@@ -337,6 +338,7 @@ constexpr unsigned kMultistepLdsReserve = 64u * 1024u;
 template <int LPR, int P, bool VEC, typename T>
 hipError_t multistep_go(const MultiParams& mp, int units, int dv, hipStream_t st) {
     constexpr int RPP = 256 / LPR;
+    if (const hipError_t e = check_grid(units, 256); e != hipSuccess) return e;
     dim3 grid(units, (dv + P * RPP - 1) / (P * RPP));
     hipLaunchKernelGGL((gdr_multistep_kernel<LPR, P, VEC, T>), grid, dim3(256), kMultistepLdsReserve, st, mp);
     return hipGetLastError();
@@ -365,6 +367,7 @@ template <bool VEC, typename T>
 hipError_t recurrent_pick_lpr(const SeqParams& sp, int units, int dk, int dv, hipStream_t st) {
     const int lpr = lanes_per_row(dk);
     const int rpw = 64 / lpr;
+    if (const hipError_t e = check_grid(units, 64); e != hipSuccess) return e;
     dim3 grid(units, (dv + rpw - 1) / rpw);
     switch (lpr) {
         case 2: hipLaunchKernelGGL((gdr_recurrent_kernel<2, VEC, T>), grid, dim3(64), 0, st, sp); break;
@@ -384,11 +387,13 @@ hipError_t staged_pick_lpr(const SeqParams& sp, int units, int dk, int dv, hipSt
         // four rows, so that two waves share each SIMD and hide each
         // other's latency along the position chain.
         using Sh = StageShape<16, 8, 8>;
+        if (const hipError_t e = check_grid(units, Sh::THREADS); e != hipSuccess) return e;
         dim3 grid(units, (dv + Sh::RPB - 1) / Sh::RPB);
         hipLaunchKernelGGL((gdr_staged_recurrent_kernel<16, T, 8, 8>), grid, dim3(Sh::THREADS), 0, st, sp, max_len);
         return hipGetLastError();
     }
     const int rpb = kStageWaves * (64 / lpr);
+    if (const hipError_t e = check_grid(units, kStageThreads); e != hipSuccess) return e;
     dim3 grid(units, (dv + rpb - 1) / rpb);
     switch (lpr) {
         case 2: hipLaunchKernelGGL((gdr_staged_recurrent_kernel<2, T, 16, kStageWaves>), grid, dim3(kStageThreads), 0, st, sp, max_len); break;

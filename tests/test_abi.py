@@ -377,3 +377,28 @@ def test_rmsnorm_validation(over, status, msg):
         setattr(a, key, val)
     assert _abi.lib().rhz_rmsnorm_heads(byref(a), None) == status
     assert msg in _abi.last_error()
+
+
+# More workgroups than a grid holds (2^32 work-items: the runtime truncates a
+# larger one without an error) are refused before the launch.
+_GRIDS = [
+    ("rhz_gdr_decode_step", lambda: _decode(batch=1 << 20, heads=16, d_k=4, d_v=4)),
+    ("rhz_gdr_multistep", lambda: _multistep(batch=1 << 20, steps=1, heads=16, d_k=4, d_v=4)),
+    ("rhz_gdr_prefill", lambda: _prefill(batch=1 << 20, seq_len=2, heads=16, d_k=8, d_v=8, algo=_abi.ALGO_CHUNKED)),
+    ("rhz_gdr_prefill", lambda: _prefill(batch=1 << 20, seq_len=2, heads=16, d_k=8, d_v=8, dtype=_abi.F32)),
+    ("rhz_gdr_prefill", lambda: _prefill(batch=1 << 19, seq_len=2, heads=16, d_k=80, d_v=8, dtype=_abi.F32)),
+    ("rhz_gdr_prefill", lambda: _prefill(batch=1 << 22, seq_len=2, heads=16, d_k=5, d_v=5, dtype=_abi.F32)),
+    ("rhz_causal_conv1d", lambda: _conv(batch=1, seq_len=1 << 28, channels=1)),
+]
+
+
+@pytest.mark.parametrize("entry,make", _GRIDS, ids=lambda x: x if isinstance(x, str) else "")
+def test_grids_beyond_the_runtime_are_refused(entry, make):
+    a = make()
+    assert getattr(_abi.lib(), entry)(byref(a), None) == _abi.ERR_HIP
+    assert "invalid configuration" in _abi.last_error(), _abi.last_error()
+
+
+def test_philox_fill_beyond_a_grid_is_refused():
+    assert _abi.lib().rhz_philox_fill(0, 1, 1, 1 << 32, 1, 0.0, 1.0, _abi.F32, A, None) == _abi.ERR_HIP
+    assert "invalid configuration" in _abi.last_error(), _abi.last_error()
