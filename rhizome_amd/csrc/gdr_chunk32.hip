@@ -70,16 +70,22 @@ constexpr int kLdV = 36;  // fp32 row stride of the V tile (4 rows apart: 16 ban
 constexpr int kLdA = 20;  // fp32 row stride of A and D
 constexpr float kKeyBetaMax = 2.0f;  // largest beta |k|^2 (the step is non-expansive up to 2)
 
-// Sequences of up to kShortLen tokens are run by the recurrence: the
-// pipeline's start costs a workgroup about 8 us, the recurrence 0.26 us per
-// token (256 units of d = 128, four workgroups per CU in turn: 59 against 52 us
-// at 64 tokens, 139 against 193 us at 256).
-constexpr int kShortLen = 64;
+// Sequences of up to short_len tokens are run by the recurrence.  The line is
+// where its time and this kernel's cross when workgroups fill the CUs several
+// times over (H = 16, d = 128, B = 16: 62 against 69 us at 80 tokens, 74
+// against 75 at 96, 100 against 86 at 128); launches that leave CUs idle would
+// cross earlier (B = 1: 22 against 17 us at 80), but a sequence's arithmetic
+// must not depend on its batch.  With d_k <= 64, where a CU takes three of the
+// recurrence's workgroups of 64 or 128 rows, the two cross late when the CUs are
+// filled many times over (d = 64, d_v = 256, B = 64: 296 against 486 us at 128
+// tokens; B = 16: 406 against 425 at 640) and early when they are not (B = 1:
+// 38 against 17 us at 128, 175 against 54 at 640): the line lies between.
+__host__ __device__ constexpr int short_len(int d_k) { return d_k > 64 ? 96 : 128; }
 
 struct Chunk32Params {
     SeqParams sp;
     int batch, units, n_tiles;
-    int long_only;  // units count the sequences of more than kShortLen tokens (the recurrence kernel runs the others)
+    int long_only;  // units count the sequences of more than short_len tokens (the recurrence kernel runs the others)
     int first;      // the launch's first workgroup
 };
 
@@ -780,7 +786,7 @@ __device__ __forceinline__ void out32(const SeqParams& p, const Unit32& u, Smem3
     }
 }
 
-// The r-th sequence of a pack (from 0) among those of more than kShortLen
+// The r-th sequence of a pack (from 0) among those of more than short_len
 // tokens, or -1.  Called by the whole workgroup; `scratch`, nine ints of LDS,
 // is free after the caller's next barrier.
 __device__ __forceinline__ int nth_long(const SeqParams& p, int batch, int r, int* scratch) {
@@ -791,7 +797,7 @@ __device__ __forceinline__ int nth_long(const SeqParams& p, int batch, int r, in
         if (s < batch) {
             int t0, t1;
             seq_bounds(p.cu_seqlens, s, p.seq_len, t0, t1);
-            is_long = t1 - t0 > kShortLen;
+            is_long = t1 - t0 > short_len(p.d_k);
         }
         const uint64_t m = __builtin_amdgcn_ballot_w64(is_long);
         if (l == 0) scratch[w] = __popcll(m);
@@ -826,7 +832,7 @@ __global__ __launch_bounds__(512, 2) void gdr_chunk32_kernel(Chunk32Params cp) {
     }
     seq_bounds(p.cu_seqlens, u.seq, p.seq_len, u.tb, u.te);
     u.nch = (u.te - u.tb + kC - 1) / kC;
-    if (u.te - u.tb <= kShortLen) {  // uniform
+    if (u.te - u.tb <= short_len(DK)) {  // uniform
         recurrence32<DK>(p, smu, u.seq, u.h, u.i0);
         return;
     }
@@ -860,7 +866,7 @@ __global__ __launch_bounds__(512, 2) void gdr_chunk32_kernel(Chunk32Params cp) {
 
 bool chunk32_supported(const rhz_gdr_prefill_args& a) {
     const auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    if (!a.cu_seqlens && a.seq_len <= kShortLen) return false;
+    if (!a.cu_seqlens && a.seq_len <= short_len(a.d_k)) return false;
     // 16-byte accesses throughout, and 32-bit byte offsets within a chunk
     return a.dtype == RHZ_F32 && a.d_k % 4 == 0 && a.d_k <= 128 && a.d_v % 4 == 0 && al16(a.q) && al16(a.k) &&
            al16(a.v) && al16(a.o) && al16(a.initial_state) && al16(a.final_state) &&
@@ -879,9 +885,10 @@ hipError_t launch_chunk32(const rhz_gdr_prefill_args& a, hipStream_t st) {
     // nothing to do, took 0.55 us per 256).  H=16 d=64, 1024 sequences of one
     // token: 227 us in one launch, 154 with empty workgroups, 87 so.  A
     // sequence's arithmetic follows from its own length in either case.
-    if (a.cu_seqlens && a.seq_len / a.batch <= kShortLen && (int64_t)cp.units * cp.n_tiles > 256) {
-        const hipError_t e = launch_staged_short(cp.sp, cp.units, kShortLen, st);
-        const int most = a.seq_len / (kShortLen + 1);
+    const int len = short_len(a.d_k);
+    if (a.cu_seqlens && a.seq_len / a.batch <= len && (int64_t)cp.units * cp.n_tiles > 256) {
+        const hipError_t e = launch_staged_short(cp.sp, cp.units, len, st);
+        const int most = a.seq_len / (len + 1);
         if (e != hipSuccess || most == 0) return e;
         cp.units = (most < a.batch ? most : a.batch) * a.heads;
         cp.long_only = 1;
