@@ -62,7 +62,7 @@ typedef enum rhz_gate { RHZ_GATE_LOG_ALPHA = 0, RHZ_GATE_ALPHA = 1 } rhz_gate;
 
 /* Prefill algorithm.  AUTO picks CHUNKED for bf16 and, for fp32, the
  * recurrence, which it applies to 16 positions at a time in fp32 to sequences
- * of more than 96 tokens (128 with d_k <= 64) where d_k <= 128, d_k and d_v are
+ * of more than 96 tokens (64 with d_k <= 32) where d_k <= 128, d_k and d_v are
  * multiples of 4 and the tensors 16-byte aligned (as accurate; a tile whose
  * inputs leave the domain below, with beta |k|^2 up to 2, is run token by
  * token).  Large fp32 batches of a few hundred tokens with d_k <= 64 are faster

@@ -70,17 +70,21 @@ constexpr int kLdV = 36;  // fp32 row stride of the V tile (4 rows apart: 16 ban
 constexpr int kLdA = 20;  // fp32 row stride of A and D
 constexpr float kKeyBetaMax = 2.0f;  // largest beta |k|^2 (the step is non-expansive up to 2)
 
-// Sequences of up to short_len tokens are run by the recurrence.  The line is
-// where its time and this kernel's cross when workgroups fill the CUs several
-// times over (H = 16, d = 128, B = 16: 62 against 69 us at 80 tokens, 74
-// against 75 at 96, 100 against 86 at 128); launches that leave CUs idle would
-// cross earlier (B = 1: 22 against 17 us at 80), but a sequence's arithmetic
-// must not depend on its batch.  With d_k <= 64, where a CU takes three of the
-// recurrence's workgroups of 64 or 128 rows, the two cross late when the CUs are
-// filled many times over (d = 64, d_v = 256, B = 64: 296 against 486 us at 128
-// tokens; B = 16: 406 against 425 at 640) and early when they are not (B = 1:
-// 38 against 17 us at 128, 175 against 54 at 640): the line lies between.
-__host__ __device__ constexpr int short_len(int d_k) { return d_k > 64 ? 96 : 128; }
+// Sequences of up to short_len tokens are run by the recurrence.  A sequence's
+// arithmetic must not depend on its batch, so the line follows from its length
+// and d_k alone, while the times cross at lengths that depend on how often the
+// launch fills the CUs.  H = 16, recurrence against this kernel, us:
+//   d_k = d_v = 128: B=16 52/68 at 65 tokens, 74/75 at 96, 100/86 at 128
+//                    B=1  19/17 at 65, 26/19 at 96
+//   d_k 64, d_v 256: B=64 155/380 at 65, 221/421 at 96, 437/636 at 192
+//                    B=16 47/97 at 65, 64/106 at 96, 406/425 at 640
+//                    B=1  22/13 at 65, 30/14 at 96, 55/21 at 192, 175/54 at 640
+//   d_k 32, d_v 128: B=64 50/92 at 65, 66/101 at 96, 126/157 at 192
+//                    B=1  20/10 at 65, 28/11 at 96, 54/16 at 192
+// At d_k > 64 the line is where full launches cross.  Below, where a CU takes
+// three of the recurrence's workgroups of 64 or 128 rows, it is where what full
+// launches lose and what the others gain are about the same factor.
+__host__ __device__ constexpr int short_len(int d_k) { return d_k > 32 ? 96 : 64; }
 
 struct Chunk32Params {
     SeqParams sp;

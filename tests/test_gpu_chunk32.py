@@ -38,11 +38,12 @@ SHAPES = [
     # mostly short sequences, in one launch
     dict(lengths=[64, 65, 0, 3, 100, 7, 1, 64, 130, 33], heads=2, d_k=128, d_v=40, state_std=0.3),
     dict(lengths=[5, 40], heads=2, d_k=32, d_v=64),
-    # just above the lengths that the recurrence keeps (96 tokens, 128 with d_k <= 64)
+    # just above the lengths that the recurrence keeps (96 tokens, 64 with d_k <= 32)
     dict(batch=1, heads=2, seq_len=97, d_k=100, d_v=52),
     dict(batch=2, heads=2, seq_len=112, d_k=128, d_v=128),
     dict(batch=1, heads=2, seq_len=113, d_k=68, d_v=36),
-    dict(batch=2, heads=3, seq_len=129, d_k=32, d_v=32),
+    dict(batch=2, heads=3, seq_len=65, d_k=32, d_v=32),
+    dict(batch=1, heads=3, seq_len=97, d_k=36, d_v=32),
     dict(batch=1, heads=2, seq_len=144, d_k=20, d_v=36),
     dict(batch=3, heads=1, seq_len=145, d_k=64, d_v=64),
     dict(batch=1, heads=5, seq_len=191, d_k=36, d_v=12),
@@ -101,12 +102,12 @@ def test_batch_invariant(device, d_k):
 @pytest.mark.parametrize("d_k,d_v", [(20, 12), (32, 96), (64, 40), (100, 64), (128, 128)])
 @pytest.mark.parametrize("tail", [0, 300])
 def test_short_sequences_are_the_recurrence(device, d_k, d_v, tail):
-    """Sequences of up to 96 tokens (128 with d_k <= 64): the same bits in a
+    """Sequences of up to 96 tokens (64 with d_k <= 32): the same bits in a
     pack, in a pack large enough for the recurrence's own launch (300 sequences
     more), in a dense batch and under RECURRENT."""
     import rhizome_amd
 
-    w = Prefill(lengths=[96 if d_k > 64 else 128, 17, 0, 1, 33, 64] + [1] * tail, heads=2, d_k=d_k, d_v=d_v, dtype=torch.float32,
+    w = Prefill(lengths=[96 if d_k > 32 else 64, 17, 0, 1, 33, 64] + [1] * tail, heads=2, d_k=d_k, d_v=d_v, dtype=torch.float32,
                 device=device, state_std=0.3)
     o, f = w.run()
     ro, rf = w.run(algo="recurrent")
@@ -119,15 +120,15 @@ def test_short_sequences_are_the_recurrence(device, d_k, d_v, tail):
 
 
 # short and long sequences in turn, more than 256 workgroups of 32 rows, and a
-# mean length of at most 96: the short ones go out in the recurrence's launch,
+# mean length of at most 64: the short ones go out in the recurrence's launch,
 # the others in the chunked one
 @pytest.mark.parametrize("d_k,d_v", [(32, 128), (64, 64), (128, 96)])
 def test_pack_in_two_launches(device, d_k, d_v):
     import rhizome_amd
 
-    lengths = [0, 1, 95, 96, 97, 200, 5, 129, 0, 70, 16, 128, 40, 0, 2, 1] * 4
+    lengths = [0, 1, 63, 64, 65, 200, 5, 97, 0, 70, 16, 96, 40, 0, 2, 1] * 4
     w = Prefill(lengths=lengths, heads=4, d_k=d_k, d_v=d_v, dtype=torch.float32, device=device, state_std=0.3)
-    assert len(lengths) * w.heads * ((d_v + 31) // 32) > 256 and w.n_tok // len(lengths) <= 96
+    assert len(lengths) * w.heads * ((d_v + 31) // 32) > 256 and w.n_tok // len(lengths) <= 64
     o, f = w.run()
     _check(w, o, f, f"two launches d_k={d_k}")
     for i in range(len(lengths) - 16, len(lengths)):
@@ -200,7 +201,7 @@ def test_out_of_domain_is_the_recurrence(device, case, in_place, d_k):
     (sequence, head) is unchanged, and the head's tiles equal the recurrence
     bit for bit or the chunked result where they hold no such value (a value
     row's tile), also when the state is updated in place."""
-    kw = dict(heads=2, d_k=d_k, d_v=64, lengths=[47, 102 if d_k > 64 else 140], dtype=torch.float32, device=device, state_std=0.1)
+    kw = dict(heads=2, d_k=d_k, d_v=64, lengths=[47, 102], dtype=torch.float32, device=device, state_std=0.1)
     w, plain = Prefill(**kw), Prefill(**kw)
     if "3e38" in case:
         w.q *= 1e3
