@@ -63,9 +63,9 @@ typedef enum rhz_gate { RHZ_GATE_LOG_ALPHA = 0, RHZ_GATE_ALPHA = 1 } rhz_gate;
 /* Prefill algorithm.  AUTO picks CHUNKED for bf16 and, for fp32, the
  * recurrence, which it applies to 16 positions at a time in fp32 to sequences
  * of more than 96 tokens (64 with d_k <= 32) where d_k <= 128, d_k and d_v are
- * multiples of 4 and the tensors 16-byte aligned (as accurate; a tile whose
- * inputs leave the domain below, with beta |k|^2 up to 2, is run token by
- * token).  Large fp32 batches of a few hundred tokens with d_k <= 64 are faster
+ * multiples of 4 and the tensors 16-byte aligned (its error is the
+ * recurrence's within a tenth; a tile whose inputs leave the domain below, with
+ * beta |k|^2 up to 2, is run token by token).  Large fp32 batches of a few hundred tokens with d_k <= 64 are faster
  * under RECURRENT.
  * RECURRENT: token-sequential fp32 recurrence.
  * CHUNKED:   64-token chunks, WY/UT transform on fp16 MFMA with fp32
