@@ -85,6 +85,8 @@ constexpr float kKeyBetaMax = 2.0f;  // largest beta |k|^2 (the step is non-expa
 // three of the recurrence's workgroups of 64 or 128 rows, it is where what full
 // launches lose and what the others gain are about the same factor.
 __host__ __device__ constexpr int short_len(int d_k) { return d_k > 32 ? 96 : 64; }
+// the roles take it that a sequence has five chunks or more, two superblocks
+static_assert(short_len(32) >= 4 * kC && short_len(128) >= 4 * kC, "every sequence here has a second superblock");
 
 struct Chunk32Params {
     SeqParams sp;
@@ -341,24 +343,22 @@ __device__ __forceinline__ void stage32(const SeqParams& p, const Unit32& u, Sme
 
 template <int DK>
 __device__ __forceinline__ void loader32(const SeqParams& p, const Unit32& u, Smem32<DK>& sm, int j) {
-    if (u.nch > 0) {
-        In32<DK> r0, r1;
-        Off32<DK> o;
-        o.set(p, u.i0, j, kC - 1);
-        load32<DK>(p, u, 0, j, o, r0);
-        load32<DK>(p, u, 1, j, o, r1);
-        for (int c = 0; c < u.nch; c += 2) {
-            stage32<DK>(p, u, sm, c, j, r0);
-            load32<DK>(p, u, c + 2, j, o, r0);
+    In32<DK> r0, r1;
+    Off32<DK> o;
+    o.set(p, u.i0, j, kC - 1);
+    load32<DK>(p, u, 0, j, o, r0);
+    load32<DK>(p, u, 1, j, o, r1);
+    for (int c = 0; c < u.nch; c += 2) {
+        stage32<DK>(p, u, sm, c, j, r0);
+        load32<DK>(p, u, c + 2, j, o, r0);
+        period_end();
+        if (c + 1 >= u.nch) break;
+        stage32<DK>(p, u, sm, c + 1, j, r1);
+        load32<DK>(p, u, c + 3, j, o, r1);
+        if (c > 0)
             period_end();
-            if (c + 1 >= u.nch) break;
-            stage32<DK>(p, u, sm, c + 1, j, r1);
-            load32<DK>(p, u, c + 3, j, o, r1);
-            if (c > 0)
-                period_end();
-            else if (period1_leaves(sm))
-                return;
-        }
+        else if (period1_leaves(sm))
+            return;
     }
     for (int i = 0; i < 4; ++i) period_end();
 }
@@ -503,22 +503,20 @@ struct TWave {
     __device__ __forceinline__ void run() {
         constexpr int HB = NB / 2;
         const int nsb = (u.nch + 3) / 4;
-        bool leave = false;  // as period1_leaves
-        if (nsb > 0) {  // superblock 0, in period 0
-            load_gates(0);
-            load_k(0, x0);
-            load_k(1, x1);
-            decays(0);
-            publish(0);
-            product(x0, 0, 2);
-            product(x1, 1, 3);
-            product(x0, 2, 4);
-            product(x1, 3, 5);
-            solve(0);
-            leave = __builtin_amdgcn_ballot_w64(bad) != 0;
-            flag32(sm, bad);
-            load_gates(1);
-        }
+        // superblock 0, in period 0
+        load_gates(0);
+        load_k(0, x0);
+        load_k(1, x1);
+        decays(0);
+        publish(0);
+        product(x0, 0, 2);
+        product(x1, 1, 3);
+        product(x0, 2, 4);
+        product(x1, 3, 5);
+        solve(0);
+        const bool leave = __builtin_amdgcn_ballot_w64(bad) != 0;  // as period1_leaves
+        flag32(sm, bad);
+        load_gates(1);
         period_end();
         const int last = u.nch + 4;  // periods in all
         for (int q = 1, sb = 1; q < last; q += 4, ++sb) {
@@ -553,8 +551,6 @@ struct TWave {
                 keep_kk(3);
                 solve(sb);
                 if (sb + 1 == nsb) flag32(sm, bad);
-            } else if (nsb == 1) {
-                flag32(sm, bad);
             }
             period_end();
         }
@@ -605,7 +601,7 @@ __device__ __forceinline__ void p_wave32(const Unit32& u, Smem32<DK>& sm, int l)
     };
     In a, b;
     period_end();
-    if (u.nch > 0) load(0, a);
+    load(0, a);
     if (period1_leaves(sm)) return;
     for (int c = 0; c < u.nch; c += 2) {  // by two, so that the operands need no copies
         step(c, a, b);
@@ -646,7 +642,7 @@ __device__ __forceinline__ void scan32(const SeqParams& p, const Unit32& u, Smem
     float finite = 0.f;
     f32x4 kx[NB];
     period_end();
-    if (u.nch > 0) load_operand<DK>(sm.k[0], sig(n), g, kx);
+    load_operand<DK>(sm.k[0], sig(n), g, kx);
     if (period1_leaves(sm)) return;
     for (int c = 0; c < u.nch; ++c) {
         const int slot = c & 3, sb = c & 7, B = c & 1;
@@ -782,7 +778,7 @@ __device__ __forceinline__ void out32(const SeqParams& p, const Unit32& u, Smem3
     period_end();
     if (period1_leaves(sm)) return;
     period_end();
-    if (u.nch > 0) load(0, a);
+    load(0, a);
     period_end();
     for (int c = 0; c < u.nch; c += 2) {
         step(c, a, b);
