@@ -15,8 +15,9 @@ rhz_gdr_local_prefill, the prefill with prepare fused in, from raw
 projections on the prefill shape, beside rhz_gdr_prepare + rhz_gdr_prefill;
 (`prefill_long_context`, `prefill_varlen`) the chunked prefill on B=1, H=32,
 T=32768, d_v=256 with slow decay, and on 64 packed sequences of 128..8192
-tokens with initial states; (`prefill_fp32`) the fp32-input path (the
-token-sequential recurrent kernel) on the headline prefill shape;
+tokens with initial states; (`prefill_fp32`) fp32 inputs on the headline
+prefill shape, as AUTO runs them (16-token chunks on fp32 MFMA), and
+(`prefill_fp32_recurrent`) the same under RECURRENT (token by token);
 (`local_chain`) the whole Local-block mixer, from the q, k, v projections
 through conv1d, prepare, the prefill and the per-head RMSNorm, in three
 arrangements of the library's calls.  Every leg first runs a settle phase of untimed
@@ -122,7 +123,8 @@ PROFILES = {
     "prepare": "prepare_kernel_bf16_t16384_h16_d128.md",
     "rmsnorm": "rmsnorm_kernel_bf16_rows262144_d128.md",
     "local": "gdr_chunk_kernel_128_pro_local_b4_h16_t4096_d128.md",
-    "prefill_fp32": "gdr_staged_recurrent_kernel_prefill_fp32_b4_h16_t4096_d128.md",
+    "prefill_fp32": "gdr_chunk32_kernel_prefill_fp32_b4_h16_t4096_d128.md",
+    "prefill_fp32_recurrent": "gdr_staged_recurrent_kernel_prefill_fp32_b4_h16_t4096_d128.md",
     "conv_prepare": "conv_prepare_kernel_bf16_t16384_h16_d128.md",
 }
 
@@ -265,18 +267,18 @@ def prefill_leg(torch, steps, warmup, c, workload, profile_key) -> dict:
             "config": {"workload": workload, **cfg},
             "roofline": {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                          "frac": gbs / PEAK_HBM_GBS, "traffic": traffic_from_profiles(profile_key),
-                         "kernel": "gdr_chunk_kernel<128, false>", "algorithmic_bytes": nbytes,
+                         "kernel": "gdr_chunk_kernel<128, false, false>", "algorithmic_bytes": nbytes,
                          "launch_us": ms * 1e3,
                          "mfma": {"achieved": tflops, "peak": PEAK_MFMA_TFLOPS, "unit": "TFLOP/s",
                                   "frac": tflops / PEAK_MFMA_TFLOPS, "flops_per_launch": flops}}}
 
 
-def bench_prefill_fp32(torch, steps, warmup) -> dict:
-    """The fp32-input path on the headline prefill shape: rhz_gdr_prefill with
-    fp32 q/k/v/o and RHZ_ALGO_RECURRENT (gdr_staged_recurrent_kernel, token by
-    token, one wave per 4 state rows of a head (16 lanes of 8 key columns per
-    row), eight waves sharing each 32-position block of k, q, gates and k.q
-    staged through LDS, two waves per SIMD)."""
+def bench_prefill_fp32(torch, steps, warmup, algo) -> dict:
+    """fp32 q/k/v/o on the headline prefill shape: algo "auto" runs them in
+    16-token chunks on fp32 MFMA (gdr_chunk32_kernel), "recurrent" token by
+    token (gdr_staged_recurrent_kernel: one wave per 4 state rows of a head, 16
+    lanes of 8 key columns per row, eight waves sharing each 32-position block
+    of k, q, gates and k.q staged through LDS, two waves per SIMD)."""
     import rhizome_amd
     from rhizome_amd import _abi, gdr
 
@@ -292,7 +294,7 @@ def bench_prefill_fp32(torch, steps, warmup) -> dict:
     g = rhizome_amd.philox_fill("neg_softplus", 0, 5, lead + (H,), f32)
     o = torch.empty(lead + (H, dv), dtype=f32, device=dev)
     fin = torch.empty((B, H, dv, dk), dtype=f32, device=dev)
-    args = gdr.prefill_args(q, k, v, g, beta, _abi.GATE_LOG_ALPHA, None, None, fin, o, "recurrent")
+    args = gdr.prefill_args(q, k, v, g, beta, _abi.GATE_LOG_ALPHA, None, None, fin, o, algo)
     stream = torch.cuda.current_stream()
     lib, argp, sp = _abi.lib(), ctypes.byref(args), ctypes.c_void_p(stream.cuda_stream or None)
 
@@ -308,26 +310,28 @@ def bench_prefill_fp32(torch, steps, warmup) -> dict:
     tokens = B * T
     nbytes = prefill_bytes(tokens, H, dk, dv, B, e_in=4, e_out=4)
     gbs = nbytes / (ms * 1e-3) / 1e9
+    recurrent = algo == "recurrent"
     # the recurrence's own arithmetic, per token-head: S k, S q and k q, the
-    # rank-1 update and o (about 8 d_k d_v multiply-adds' worth; fp32 VALU)
+    # rank-1 update and o (about 8 d_k d_v multiply-adds' worth)
     flops = float(tokens * H * 8 * dk * dv)
-    return {"metric": "GDR prefill tokens/s, fp32 inputs", "value": tokens / (ms * 1e-3), "unit": "tokens/s",
-            "ms_per_step": ms, "steps": steps, "warmup": warmup, **info,
-            "config": {"workload": "recurrent GDR prefill, fp32 q/k/v/o", "batch": B, "heads": H,
-                       "seq_len": T, "d_k": dk, "d_v": dv, "inputs": "fp32 q/k/v, fp32 log-decay and beta",
-                       "state": "fp32"},
-            # token-sequential: every wave walks the T positions of its head
-            # one after the other, so the launch is bound by the per-position
-            # latency of that chain, not by HBM
-            "latency": {"ns_per_position": ms * 1e6 / T, "positions_per_wave": T,
-                        "waves": B * H * ((dv + 3) // 4)},
-            "roofline": {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                         "frac": gbs / PEAK_HBM_GBS, "traffic": traffic_from_profiles("prefill_fp32"),
-                         "kernel": "gdr_staged_recurrent_kernel<16,float,8,8>", "algorithmic_bytes": nbytes,
-                         "launch_us": ms * 1e3,
-                         "fp32_valu": {"achieved": flops / (ms * 1e-3) / 1e12, "peak": PEAK_FP32_TFLOPS,
-                                       "unit": "TFLOP/s",
-                                       "frac": flops / (ms * 1e-3) / 1e12 / PEAK_FP32_TFLOPS}}}
+    leg = {"metric": "GDR prefill tokens/s, fp32 inputs", "value": tokens / (ms * 1e-3), "unit": "tokens/s",
+           "ms_per_step": ms, "steps": steps, "warmup": warmup, **info,
+           "config": {"workload": f"{'recurrent' if recurrent else 'chunked'} GDR prefill, fp32 q/k/v/o", "batch": B,
+                      "heads": H, "seq_len": T, "d_k": dk, "d_v": dv, "algo": algo,
+                      "inputs": "fp32 q/k/v, fp32 log-decay and beta", "state": "fp32"},
+           "roofline": {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
+                        "frac": gbs / PEAK_HBM_GBS,
+                        "traffic": traffic_from_profiles("prefill_fp32_recurrent" if recurrent else "prefill_fp32"),
+                        "kernel": "gdr_staged_recurrent_kernel<16,float,8,8>" if recurrent else
+                                  "gdr_chunk32_kernel<128>",
+                        "algorithmic_bytes": nbytes, "launch_us": ms * 1e3,
+                        "fp32": {"achieved": flops / (ms * 1e-3) / 1e12, "peak": PEAK_FP32_TFLOPS,
+                                 "unit": "TFLOP/s", "frac": flops / (ms * 1e-3) / 1e12 / PEAK_FP32_TFLOPS}}}
+    if recurrent:
+        # every wave walks the T positions of its head one after the other, so
+        # the launch is bound by the per-position latency of that chain
+        leg["latency"] = {"ns_per_position": ms * 1e6 / T, "positions_per_wave": T, "waves": B * H * ((dv + 3) // 4)}
+    return leg
 
 
 def bench_decode(torch, warmup, c=None):
@@ -550,7 +554,7 @@ def bench_local(torch, steps, warmup):
             "ms_per_step": out["fused"]["ms_per_step"],
             "roofline": {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                          "frac": gbs / PEAK_HBM_GBS, "traffic": traffic_from_profiles("local"),
-                         "kernel": "gdr_chunk_kernel<128, true>", "bytes_per_launch": nbytes,
+                         "kernel": "gdr_chunk_kernel<128, true, false>", "bytes_per_launch": nbytes,
                          "launch_us": out["fused"]["ms_per_step"] * 1e3},
             "separate_ms_per_step": out["separate"]["ms_per_step"],
             "separate_tokens_per_s": tokens / (out["separate"]["ms_per_step"] * 1e-3),
@@ -772,7 +776,8 @@ def main() -> int:
     mms, mbytes, ms_info = bench_multistep(torch, min(args.steps, 50), min(args.warmup, 20))
     aux = bench_aux(torch, min(args.steps, 50), min(args.warmup, 20))
     local = bench_local(torch, min(args.steps, 50), min(args.warmup, 10))
-    fp32_leg = bench_prefill_fp32(torch, min(args.steps, 20), min(args.warmup, 5))
+    fp32_leg = bench_prefill_fp32(torch, min(args.steps, 20), min(args.warmup, 5), "auto")
+    fp32_rec_leg = bench_prefill_fp32(torch, min(args.steps, 20), min(args.warmup, 5), "recurrent")
     chain = bench_local_chain(torch, min(args.steps, 30), min(args.warmup, 5))
     long_leg = prefill_leg(torch, min(args.steps, 50), min(args.warmup, 10), PREFILL_LONG,
                            "chunked GDR prefill, long context, slow decay", "prefill_long")
@@ -814,7 +819,7 @@ def main() -> int:
         # is reported beside it.
         "roofline": {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": gbs / PEAK_HBM_GBS, "traffic": traffic,
-                     "kernel": "gdr_chunk_kernel<128, false>", "algorithmic_bytes": algo_bytes,
+                     "kernel": "gdr_chunk_kernel<128, false, false>", "algorithmic_bytes": algo_bytes,
                      "launch_us": ms * 1e3,
                      "mfma": {"achieved": achieved, "peak": PEAK_MFMA_TFLOPS, "unit": "TFLOP/s",
                               "frac": achieved / PEAK_MFMA_TFLOPS, "flops_per_launch": flops}},
@@ -858,6 +863,7 @@ def main() -> int:
         "prologue_epilogue": aux,
         "local_block": local,
         "prefill_fp32": fp32_leg,
+        "prefill_fp32_recurrent": fp32_rec_leg,
         "local_chain": chain,
         "device": device_info(torch),
     }
