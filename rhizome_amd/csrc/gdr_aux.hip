@@ -610,8 +610,8 @@ hipError_t pick_rows(const P& p, int rows, int n, bool vec, hipStream_t st) {
 // other, where that does not cost more than it gives:
 // - With carried states every further sequence of a span is another round
 //   trip (4096 sequences of one token, 6144 bf16 channels, conv1d: 208 us in
-//   spans of one token, 292 in spans of 16; 64 sequences, conv_prepare: 9.4
-//   and 62).  Only blocks of less than half a wave of channels are bound by
+//   spans of one token, 292 in spans of 16; 64 sequences, conv_prepare: 10 and
+//   32).  Only blocks of less than half a wave of channels are bound by
 //   their number beyond 8192 (32768 sequences, 64 channels: 62 and 50 us).
 // - Without states a span's next sequence costs nothing, and each block reads
 //   20 bytes of weights and bias per channel: spans of less than 32 bytes per

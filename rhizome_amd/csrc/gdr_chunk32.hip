@@ -31,8 +31,7 @@
 //
 // Measured, B = 4 H = 16 T = 4096 d = 128: 429 us (85 TFLOP/s of fp32 MFMA, 55 %
 // of what a large fp32 matrix product reaches) against 1066 us for the
-// token-by-token kernel; a period takes about 3600 cycles on the fullest SIMD,
-// 2176 of them MFMA.
+// token-by-token kernel; a period takes about 3880 cycles, 2176 of them MFMA.
 //
 // One workgroup of 8 waves per (sequence, head, 32 rows of S), in lockstep:
 // one barrier per chunk, every wave at its own stage of the pipeline:
@@ -882,9 +881,11 @@ hipError_t launch_chunk32(const rhz_gdr_prefill_args& a, hipStream_t st) {
     // workgroups share a CU where this kernel's LDS leaves room for one, and the
     // rest here, in as many workgroups as its tokens could need (each finds its
     // sequence by counting; workgroups for every sequence, most of them with
-    // nothing to do, took 0.55 us per 256).  H=16 d=64, 1024 sequences of one
-    // token: 227 us in one launch, 154 with empty workgroups, 87 so.  A
-    // sequence's arithmetic follows from its own length in either case.
+    // nothing to do, took 0.55 us per 256).  H=16 d=64: 1024 sequences of one
+    // token 227 us in one launch, 154 with empty workgroups, 87 so; 16 of 64
+    // tokens, 512 workgroups, 39 and 26 us in one and two launches, with one of
+    // 97 to 99 tokens among them 43 and 45.  A sequence's arithmetic follows from
+    // its own length in either case.
     const int len = short_len(a.d_k);
     if (a.cu_seqlens && a.seq_len / a.batch <= len && (int64_t)cp.units * cp.n_tiles > 256) {
         const hipError_t e = launch_staged_short(cp.sp, cp.units, len, st);

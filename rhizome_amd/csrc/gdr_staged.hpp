@@ -1,7 +1,7 @@
 // gdr_staged.hpp -- the token-sequential fp32 recurrence over a block of
 // state rows, with the positions staged through LDS.  Used by
-// gdr_staged_recurrent_kernel (the fp32-input prefill) and by the chunked
-// kernel's exact rerun of a tile whose inputs leave the fp16 path's domain.
+// gdr_staged_recurrent_kernel, by the fp32 chunked kernel for short sequences,
+// and by both chunked kernels for a tile whose inputs leave their domain.
 //
 // Rows of S are independent (row i only reads v_i and its own row), so each
 // row goes to a group of LPR lanes; lane li of a group holds columns

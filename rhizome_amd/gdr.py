@@ -37,7 +37,7 @@ def _stream(stream) -> int | None:
     if stream is None:
         # the current stream's handle without a Stream object around it, for
         # calls that the host bounds (with _empty's allocations, one decode
-        # position of one sequence: 10.4 -> 7.3 us a call)
+        # position of one sequence: 10.4 -> 7.8 us a call)
         return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()) or None
     return stream.cuda_stream or None
 
